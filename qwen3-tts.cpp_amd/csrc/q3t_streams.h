@@ -138,7 +138,10 @@ __device__ __forceinline__ bool splitk_exchange(double (&acc)[NV], const GemmArg
         return false;
     }
     bool dead = false;
-    constexpr int CH = NV < 8 ? NV : 8;          // values summed per pass over the slices
+    // values summed per pass over the slices: a divisor of NV (12 values with
+    // three 16-row tiles), so that no pass reads past a slice's words
+    constexpr int CH = NV % 8 == 0 ? 8 : NV % 6 == 0 ? 6 : 4;
+    static_assert(NV % CH == 0, "whole passes");
 #pragma unroll
     for (int c0 = 0; c0 < NV; c0 += CH) {
         double tot[CH];

@@ -252,3 +252,13 @@ def test_streams_full_q8_4_streams():
         _run(cfg, dev, o, specs, chunk=8)
     finally:
         dev.close()
+
+
+@pytest.mark.parametrize("n", [17, 24, 32])
+def test_streams_three_and_four_row_tiles(tiny_q8, n):
+    """17 to 24 streams: the code predictor's 2-token prefill is 34 to 48 rows
+    (three 16-row tiles, whose split-K exchange holds 12 values a lane), 32
+    streams 64 rows (four)."""
+    cfg, w, dev, o = tiny_q8
+    specs = [dict(seed_prompt=100 + b, n_text=9 + b % 5, max_len=3, temperature=0.0, top_k=0) for b in range(n)]
+    _run(cfg, dev, o, specs, chunk=3)
