@@ -111,6 +111,11 @@ struct q3t_dev {
     // split-K partials and per-tile tickets, one set per GEMM call type
     // (QKV, Wo, gate/up, down): a set's tickets advance by S per launch
     uint64_t * spart[4] = {}; uint32_t * scnt[4] = {}; int32_t * serr = nullptr;
+    // short prefills and text projections on the few-row GEMMs: the same per
+    // call site, row sums of squares and scales, and the mapped error flag
+    uint64_t * rw_part[6] = {}; uint32_t * rw_cnt[6] = {}; int32_t * rw_err = nullptr;
+    double * rw_ss[2] = {nullptr, nullptr}; float * rw_rs = nullptr;
+    bool rw_ready = false;
     hipGraphExec_t s_exec = nullptr; hipGraph_t s_graph = nullptr;
     bool s_hm = false;            // F16 layers: the fp16-MFMA decode GEMMs (else the exact f64-MFMA ones)
     int32_t s_launched = 0, s_max = 0; bool s_ready = false;
@@ -1225,6 +1230,7 @@ void q3t_dev_destroy(q3t_dev * c) {
     for (hipEvent_t e : c->run_ev) if (e) (void) hipEventDestroy(e);
     for (void * p : c->allocs) (void) hipFree(p);
     if (c->pin) (void) hipHostFree(c->pin);
+    if (c->rw_err) (void) hipHostFree(c->rw_err);
     if (c->up_host) (void) hipHostFree(c->up_host);
     if (c->stream) (void) hipStreamDestroy(c->stream);
     delete c;
@@ -1545,11 +1551,206 @@ int q3t_dev_kv_write(q3t_dev * c, int32_t layer, int32_t n_pos, const uint16_t *
 
 namespace {
 
+// ------------------------------------------------------ few-row Q8_0 GEMMs
+// The shapes of few-row GEMM a layer needs (ms::k_gemm_sk; multi-stream decode
+// and short prefills):
+//   QKV      RMSNorm'd fp32 rows quantised in registers, fp32 out
+//   PROJ     pre-quantised rows in (attention / SwiGLU output), + residual
+//   GATE_UP  RMSNorm'd rows, gate and up matrices, SwiGLU, Q8_0 out
+// and a text projection (fp32 rows quantised in registers):
+//   FC1      + bias, SiLU          FC2      + bias
+enum GemmKind { G_QKV = 0, G_PROJ = 1, G_GATE_UP = 2, G_FC1 = 3, G_FC2 = 4 };
+constexpr int kGemmKinds = 5;
+// preferred K splits and the Q8_0 blocks per wave they leave (QKV and gate/up:
+// 32 blocks / (4 waves x 2); Wo / down: 64 or 96 / (4 x 4)).  Measured with
+// 16 streams on one box: {2, 4, 2} 2,567 aggregate frames/s, {2, 2, 2} 2,500,
+// the former {4, 8, 4} 2,340, no split {1, 1, 1} 2,051.
+constexpr int kGemmKB[kGemmKinds] = {4, 6, 4, 4, 4};       // max Q8_0 blocks per wave
+constexpr int kGemmMT[kGemmKinds] = {1, 1, 2, 1, 1};       // 16-row tiles per workgroup
+constexpr int kGemmS[kGemmKinds] = {2, 4, 2, 4, 4};        // preferred K splits
+
+template <int NT, int KIND>
+const void * gemm_kernel() {
+    if (KIND == G_QKV) return (const void *) ms::k_gemm_sk<NT, 1, false, ms::IN_NORM, ms::OUT_F32, kGemmKB[G_QKV]>;
+    if (KIND == G_PROJ) return (const void *) ms::k_gemm_sk<NT, 1, false, ms::IN_Q8, ms::OUT_RESID, kGemmKB[G_PROJ]>;
+    if (KIND == G_FC1) return (const void *) ms::k_gemm_sk<NT, 1, false, ms::IN_PLAIN, ms::OUT_BIAS_SILU, kGemmKB[G_FC1]>;
+    if (KIND == G_FC2) return (const void *) ms::k_gemm_sk<NT, 1, false, ms::IN_PLAIN, ms::OUT_RESID, kGemmKB[G_FC2]>;
+    return (const void *) ms::k_gemm_sk<NT, 2, true, ms::IN_NORM, ms::OUT_SWIGLU_Q8, kGemmKB[G_GATE_UP]>;
+}
+
+template <int KIND>
+const void * gemm_kernel_nt(int nt) {
+    switch (nt) {
+        case 1: return gemm_kernel<1, KIND>();
+        case 2: return gemm_kernel<2, KIND>();
+        case 3: return gemm_kernel<3, KIND>();
+        default: return gemm_kernel<4, KIND>();
+    }
+}
+
+const void * gemm_fn(int kind, int nt) {
+    switch (kind) {
+        case G_QKV: return gemm_kernel_nt<G_QKV>(nt);
+        case G_PROJ: return gemm_kernel_nt<G_PROJ>(nt);
+        case G_FC1: return gemm_kernel_nt<G_FC1>(nt);
+        case G_FC2: return gemm_kernel_nt<G_FC2>(nt);
+        default: return gemm_kernel_nt<G_GATE_UP>(nt);
+    }
+}
+
+// K splits for a contraction of nb Q8_0 blocks that leave at most KB blocks
+// per wave: the kind's preference, else more (up to 8, wider models), else
+// fewer; 0 if none.
+int gemm_splits(int kind, int nb) {
+    const auto ok = [&](int S) { return nb % (ms::kWaves * S) == 0 && nb / (ms::kWaves * S) <= kGemmKB[kind]; };
+    for (int S = kGemmS[kind]; S <= 8; S *= 2)
+        if (ok(S)) return S;
+    for (int S = kGemmS[kind] / 2; S >= 1; S /= 2)
+        if (ok(S)) return S;
+    return 0;
+}
+
+size_t gemm_lds(int kind, int nt, int K) {
+    const int S = gemm_splits(kind, K / kQK);
+    return ms::gemm_sk_lds_bytes(nt, kGemmMT[kind], kind == G_GATE_UP, S ? K / kQK / S : 0);
+}
+
+// tagged words of the partials one launch may store: tiles x S x 2 per value x values per lane x 64 lanes
+size_t gemm_part_words(int kind, int nt, int N, int K) {
+    const int mt = kGemmMT[kind], nw = kind == G_GATE_UP ? 2 : 1;
+    return (size_t) (N / (ms::kRows * mt)) * gemm_splits(kind, K / kQK) * 2 * nw * mt * nt * 4 * 64;
+}
+
+// One launch; part / cnt: the call site's partials and tickets, whose launches
+// all use the same split count.
+void gemm_sk(q3t_dev * c, int kind, ms::GemmArgs a, uint64_t * part, uint32_t * cnt, int32_t * err) {
+    const int nt = (a.n + 15) / 16;
+    const int S = gemm_splits(kind, a.K / kQK);
+    a.part = part; a.cnt = cnt; a.err = err;
+    void * args[] = {(void *) &a};
+    (void) hipLaunchKernel(gemm_fn(kind, nt), dim3(a.N / (ms::kRows * kGemmMT[kind]), S), dim3(ms::kThreads), args,
+                           gemm_lds(kind, nt, a.K), c->stream);
+}
+
+// Allows the few-row GEMMs all of the device's LDS (their dynamic LDS depends
+// on the contraction, and contexts of different widths share the kernels).
+hipError_t allow_gemm_lds(int max_lds) {
+    for (int kind = 0; kind < kGemmKinds; ++kind)
+        for (int nt = 1; nt <= 4; ++nt) {
+            const hipError_t e =
+                hipFuncSetAttribute(gemm_fn(kind, nt), hipFuncAttributeMaxDynamicSharedMemorySize, max_lds);
+            if (e != hipSuccess) return e;
+        }
+    return hipSuccess;
+}
+
+// RMSNorm row scales of n rows of width K.
+void row_scales(q3t_dev * c, const float * x, int xs, int K, int n, float * out) {
+    hipLaunchKernelGGL(ms::k_row_scale, dim3(n), dim3(kBlock), 0, c->stream, x, xs, K, c->cfg.rms_eps, out);
+}
+
+// ---------------------------------------------------------- short prefills
+// Up to kRowsMax prompt rows of a Q8_0 model take the multi-stream decode's
+// layer program, the rows of the one prompt in the place of the streams: four
+// few-row GEMMs (RMSNorm, quantisation, residual and SwiGLU inside), the K/V
+// rows, and the 16-wave decode attention with one workgroup per (row, head),
+// 6 launches a layer instead of 11, the same numbers.  Bound by its chain of
+// launches; each 16-row tile adds its weights' fp64 scale work.  Measured on
+// the 0.6B shapes (ms, this / the tiled prefill / GEMV chunks), no history:
+// 2 rows 1.39 / 4.27 / 1.17, 3 rows 1.39 / 4.29 / 2.06, 10 rows 1.44 / 4.34 /
+// 5.80, 32 rows 2.08 / 4.56 / 18.5, 64 rows 3.42 / 4.93 / 37.3; behind 1,000
+// cached positions: 2 rows 1.77 / 8.02 / 2.88, 10 rows 1.81 / 8.02 / 10.7,
+// 64 rows 4.84 / 7.70 / 63.2.  The GEMM's column tiles end at 64 rows; two
+// 64-row passes would take 6.8 ms where the tiled prefill of 96 rows takes 5.3.
+constexpr int kRowsMax = 64;
+constexpr int kRowsTwo = 160;   // 2 rows: from this many cached positions (GEMV chunks add 1.7 us each, this 0.4)
+
+// Call sites of the short prefill and of the text projection: each has its
+// own tickets and partials (a site's launches all split K alike).
+enum RowsSite { R_QKV = 0, R_WO = 1, R_GATE_UP = 2, R_DOWN = 3, R_FC1 = 4, R_FC2 = 5, kRowsSites = 6 };
+struct RowsShape { int kind, N, K; };
+
+RowsShape rows_shape(const q3t_config & g, int site) {
+    const int d = g.hidden_size, qd = g.n_head * g.head_dim, kd = g.n_kv_head * g.head_dim, te = g.text_embd_dim;
+    switch (site) {
+        case R_QKV: return {G_QKV, qd + 2 * kd, d};
+        case R_WO: return {G_PROJ, d, qd};
+        case R_GATE_UP: return {G_GATE_UP, g.ffn_size, d};
+        case R_DOWN: return {G_PROJ, d, g.ffn_size};
+        case R_FC1: return {G_FC1, te, te};
+        default: return {G_FC2, d, te};
+    }
+}
+
+bool rows_site_ok(const q3t_config & g, int site) {
+    const RowsShape s = rows_shape(g, site);
+    return s.K % kQK == 0 && s.N % (ms::kRows * kGemmMT[s.kind]) == 0 && gemm_splits(s.kind, s.K / kQK) > 0;
+}
+
+// Tickets, partials, row sums and the wait error flag (mapped host memory, so
+// reading it costs no copy).  Zeroed here: tickets and tags start at 0.
+int ensure_rows(q3t_dev * c) {
+    if (c->rw_ready) return 0;
+    const q3t_config & g = c->cfg;
+    int max_lds = 0;
+    HIP_OK(hipDeviceGetAttribute(&max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, c->device));
+    HIP_OK(allow_gemm_lds(max_lds));
+    for (int i = 0; i < kRowsSites; ++i) {
+        const RowsShape s = rows_shape(g, i);
+        if (!rows_site_ok(g, i)) continue;
+        const size_t words = gemm_part_words(s.kind, kRowsMax / 16, s.N, s.K), tiles = (size_t) s.N / ms::kRows;
+        if (!c->rw_part[i] && dev_alloc_t(c, &c->rw_part[i], words)) return -1;
+        if (!c->rw_cnt[i] && dev_alloc_t(c, &c->rw_cnt[i], tiles)) return -1;
+        HIP_OK(hipMemsetAsync(c->rw_part[i], 0, words * 8, c->stream));
+        HIP_OK(hipMemsetAsync(c->rw_cnt[i], 0, tiles * sizeof(uint32_t), c->stream));
+    }
+    for (int i = 0; i < 2; ++i)
+        if (!c->rw_ss[i] && dev_alloc_t(c, &c->rw_ss[i], (size_t) kRowsMax * (g.hidden_size / ms::kRows))) return -1;
+    if (!c->rw_rs && dev_alloc_t(c, &c->rw_rs, (size_t) kRowsMax)) return -1;
+    if (!c->rw_err) HIP_OK(hipHostMalloc((void **) &c->rw_err, sizeof(int32_t), hipHostMallocMapped));
+    *c->rw_err = 0;
+    c->rw_ready = true;
+    return 0;
+}
+
+void rows_gemm(q3t_dev * c, int site, ms::GemmArgs a) {
+    const RowsShape s = rows_shape(c->cfg, site);
+    a.N = s.N; a.K = s.K;
+    gemm_sk(c, s.kind, a, c->rw_part[site], c->rw_cnt[site], c->rw_err);
+}
+
+// After a synchronisation: a split-K partial of this call never arrived.
+int rows_check(q3t_dev * c) {
+    if (!c->rw_err || !*c->rw_err) return 0;
+    *c->rw_err = 0;
+    c->rw_ready = false;              // tickets of unfinished launches: start over from zero
+    return fail(c, "short prefill: a split-K partial never arrived (device wait timed out)");
+}
+
+// Which prefills take it: all layers Q8_0, at most kRowsMax rows, and an
+// attention launch whose LDS holds a row's scores.  Q3T_PREFILL_MFMA (either
+// value) keeps the other paths.
+bool rows_prefill(q3t_dev * c, int n, int n_past) {
+    if (n < (n_past < kRowsTwo ? 3 : 2) || n > kRowsMax || std::getenv("Q3T_PREFILL_MFMA") || !c->gqa_lds_ok)
+        return false;
+    const q3t_config & g = c->cfg;
+    if (g.head_dim != kHD || g.n_head % g.n_kv_head || g.hidden_size % (4 * ms::kRows)) return false;
+    for (int s : {(int) R_QKV, (int) R_WO, (int) R_GATE_UP, (int) R_DOWN})
+        if (!rows_site_ok(g, s)) return false;
+    for (int i = 0; i < g.n_layers; ++i) {
+        const LayerDev & L = c->talker[i];
+        for (const Slot * w : {&L.qkv, &L.wo, &L.wg, &L.wu, &L.wd})
+            if (w->type != Q3T_TYPE_Q8_0) return false;
+    }
+    return true;
+}
+
 // Which tiled path the talker prefill of n tokens takes: 1 = int8 MFMA GEMMs
 // (Q8_0 layers), 2 = exact F16 VALU GEMMs (F16 layers), 0 = the chunked GEMV
-// prefill.  Tiled needs GEMM-friendly widths and, measured on the 0.6B shapes,
-// pays from 9 rows for Q8_0 (10 rows: 5.2 ms against 5.8 ms in 4-row GEMV
-// chunks) and from 40 rows for F16 (its VALU tiles take ~22 ms for any n up to
+// prefill.  Short Q8_0 prefills go elsewhere first (rows_prefill).  Tiled needs
+// GEMM-friendly widths and, measured on the 0.6B shapes, pays from 9 rows for
+// Q8_0 (10 rows: 4.3 ms against 5.8 ms in 4-row GEMV chunks) and from 40 rows
+// for F16 (its VALU tiles take ~22 ms for any n up to
 // 64, the GEMV ~2.3 ms per 4 rows).  Q3T_PREFILL_MFMA=0 disables it, =1 uses
 // it for any n.
 int tiled_prefill(q3t_dev * c, int n) {
@@ -1896,6 +2097,64 @@ int prefill_mfma(q3t_dev * c, int n, int n_past) {
     return 0;
 }
 
+// Talker prefill of n <= kRowsMax tokens (rows in c->stage) on the few-row
+// GEMMs; buffers and outputs as prefill_mfma.
+int prefill_rows(q3t_dev * c, int n, int n_past) {
+    const q3t_config & g = c->cfg;
+    const int d = g.hidden_size, qd = g.n_head * g.head_dim, kd = g.n_kv_head * g.head_dim, qkvd = qd + 2 * kd;
+    const size_t lstride = (size_t) g.n_kv_head * c->n_ctx * g.head_dim;
+    const int tiles = d / ms::kRows;
+    const float * x = c->stage;
+    row_scales(c, x, d, d, n, c->rw_rs);
+    for (int il = 0; il < g.n_layers; ++il) {
+        const LayerDev & L = c->talker[il];
+        uint16_t * kc = c->kc + il * lstride;
+        uint16_t * vc = c->vc + il * lstride;
+        ms::GemmArgs q{};
+        q.W = (const int8_t *) L.qkv.data; q.Wd = L.qkv.scales;
+        q.x = x; q.xs = d; q.rscale = c->rw_rs; q.norm_w = L.attn_norm; q.n = n; q.y = c->pf_qkv; q.ys = qkvd;
+        if (il > 0) { q.ss_in = c->rw_ss[1]; q.ss_tiles = tiles; q.eps = g.rms_eps; }
+        rows_gemm(c, R_QKV, q);
+        hipLaunchKernelGGL(pf::k_kv_rows, dim3(n, (g.n_kv_head + 3) / 4), dim3(kBlock), 0, c->stream, (const float *) c->pf_qkv,
+                           qkvd, qd, kd, L.k_norm, g.rms_eps, (const float *) c->rope_cos, (const float *) c->rope_sin,
+                           kc, vc, c->n_ctx, n_past, c->kv_bf16 ? 1 : 0);
+        ms::GqaArgs at{};
+        at.qkv = c->pf_qkv; at.qkv_stride = qkvd;
+        at.q_norm = L.q_norm; at.k_norm = L.k_norm; at.eps = g.rms_eps;
+        at.rope_cos = c->rope_cos; at.rope_sin = c->rope_sin;
+        at.kc = kc; at.vc = vc; at.n_ctx = c->n_ctx; at.n_head = g.n_head; at.n_kv_head = g.n_kv_head;
+        at.pos_const = n_past; at.pos_row = 1; at.no_append = 1;
+        at.out = c->pf_att; at.out_stride = qd; at.out_q = c->pf_q; at.out_dx = c->pf_dx;
+        at.scale = 1.0f / std::sqrt((float) g.head_dim);
+        const dim3 grid(g.n_head, n), block(ms::kAThreads);
+        const size_t al = ms::attn_gqa_lds_bytes(1, n_past + n);
+        if (c->kv_bf16) hipLaunchKernelGGL((ms::k_attn_gqa<1, true>), grid, block, al, c->stream, at);
+        else hipLaunchKernelGGL(ms::k_attn_gqa<1>, grid, block, al, c->stream, at);
+        ms::GemmArgs o{};
+        o.W = (const int8_t *) L.wo.data; o.Wd = L.wo.scales;
+        o.q = c->pf_q; o.qdx = c->pf_dx; o.n = n; o.y = c->pf_xb; o.ys = d; o.res = x; o.rs = d; o.ss_out = c->rw_ss[0];
+        rows_gemm(c, R_WO, o);
+        ms::GemmArgs f{};
+        f.W = (const int8_t *) L.wg.data; f.Wd = L.wg.scales; f.W2 = (const int8_t *) L.wu.data; f.W2d = L.wu.scales;
+        f.x = c->pf_xb; f.xs = d; f.norm_w = L.ffn_norm; f.n = n;
+        f.ss_in = c->rw_ss[0]; f.ss_tiles = tiles; f.eps = g.rms_eps;
+        f.yq = c->pf_q; f.ydx = c->pf_dx;
+        rows_gemm(c, R_GATE_UP, f);
+        ms::GemmArgs dn{};
+        dn.W = (const int8_t *) L.wd.data; dn.Wd = L.wd.scales;
+        dn.q = c->pf_q; dn.qdx = c->pf_dx; dn.n = n; dn.y = c->pf_xa; dn.ys = d; dn.res = c->pf_xb; dn.rs = d;
+        dn.ss_out = c->rw_ss[1];
+        rows_gemm(c, R_DOWN, dn);
+        x = c->pf_xa;
+    }
+    GemvSpec h{};
+    h.w = weight_of(c->codec_head); h.rows = g.codec_vocab; h.K = d;
+    h.x = c->pf_xa + (size_t) (n - 1) * d; h.x_stride = d; h.norm_w = (const float *) c->out_norm.data;
+    h.hidden_out = c->hidden; h.hidden_stride = d; h.y = c->logits; h.y_stride = g.codec_vocab;
+    gemv(c, h, 1);
+    return 0;
+}
+
 // y [n][N] = x [n][K] . W^T + bias on the tiled GEMMs (Q8_0: quantised rows on
 // int8 MFMA; F16: the exact VALU GEMM, x rounded to fp16): the GEMV's
 // EPI_BIAS, with the bias as a residual of row stride 0.
@@ -1921,16 +2180,27 @@ bool text_proj_tiled(const q3t_dev * c, int n) {
 
 // project_text_tokens (src/tts_transformer.cpp:963-1028) of n ids into the
 // device rows dst [n][d]: text_embd rows -> fc1 + bias -> SiLU -> fc2 + bias.
-// n >= 16 runs the tiled GEMMs, fewer rows the GEMV in chunks of up to 4;
-// rows are independent and both forms keep one numerics contract, so a row's
-// result does not depend on n.  ids are range-checked by the caller.
+// Q8_0: 2 to 64 rows run the few-row GEMMs (text_proj_few); else n >= 16 runs
+// the tiled GEMMs, fewer rows the GEMV in chunks of up to 4; rows are
+// independent and every form keeps one numerics contract, so a row's result
+// does not depend on n.  ids are range-checked by the caller.
 // Work buffers of one text projection of n ids: the ids on the device,
 // the gathered text_embd rows [n][te], the fc1 output (tiled: [n][te]; GEMV:
 // [4][te]) and the Q8_0 copies of the tiled GEMMs' input rows ([n][te] int8,
 // [n][te/32] scales).
 struct ProjWork {
     const int32_t * ids; float * rows; float * h; int8_t * q; float * dx;
+    bool few = false;      // both linears on the few-row GEMMs (text_proj_few)
 };
+
+// 2 to kRowsMax ids of Q8_0 text tensors take the few-row GEMMs: two launches,
+// the bias and the SiLU in their epilogues.  Measured (0.6B shapes, us a
+// call, this / tiled / GEMV chunks): 2 ids 45 / 110 / 45, 9 ids 46 / 119 / 138,
+// 32 ids 57 / 124 / 343, 64 ids 80 / 130 / 629; 65 ids tiled 133.
+bool text_proj_few(const q3t_dev * c, int n) {
+    return n >= 2 && n <= kRowsMax && !std::getenv("Q3T_PREFILL_MFMA") && c->fc1.type == Q3T_TYPE_Q8_0 &&
+           c->fc2.type == Q3T_TYPE_Q8_0 && rows_site_ok(c->cfg, R_FC1) && rows_site_ok(c->cfg, R_FC2);
+}
 
 int proj_tensors_ok(q3t_dev * c) {
     if (!c->text_embd.data || !c->fc1.data || !c->fc1_b.data || !c->fc2.data || !c->fc2_b.data)
@@ -1945,7 +2215,16 @@ void project_rows_core(q3t_dev * c, int32_t n, const ProjWork & w, float * dst) 
     const int te = g.text_embd_dim, d = g.hidden_size;
     hipLaunchKernelGGL(k_gather_rows, dim3((te + 255) / 256, n), dim3(256), 0, c->stream,
                        (const uint16_t *) c->text_embd.data, (int64_t) te, w.ids, n, w.rows);
-    if (text_proj_tiled(c, n)) {
+    if (w.few) {
+        ms::GemmArgs a{};
+        a.W = (const int8_t *) c->fc1.data; a.Wd = c->fc1.scales; a.x = w.rows; a.xs = te; a.n = n;
+        a.y = w.h; a.ys = te; a.res = (const float *) c->fc1_b.data; a.rs = 0;
+        rows_gemm(c, R_FC1, a);
+        ms::GemmArgs b{};
+        b.W = (const int8_t *) c->fc2.data; b.Wd = c->fc2.scales; b.x = w.h; b.xs = te; b.n = n;
+        b.y = dst; b.ys = d; b.res = (const float *) c->fc2_b.data; b.rs = 0;
+        rows_gemm(c, R_FC2, b);
+    } else if (text_proj_tiled(c, n)) {
         pf_linear_bias(c, c->fc1, te, te, n, w.rows, c->fc1_b, w.h, w.q, w.dx);
         const size_t cnt = (size_t) n * te;
         hipLaunchKernelGGL(k_silu_rows, dim3((unsigned) std::min<size_t>((cnt + 255) / 256, 4096)), dim3(256), 0,
@@ -1983,14 +2262,17 @@ int project_rows(q3t_dev * c, const int32_t * tokens, int32_t n, float * dst) {
     const int te = g.text_embd_dim;
     HIP_OK(hipMemcpyAsync(c->ids, tokens, (size_t) n * 4, hipMemcpyHostToDevice, c->stream));
     ProjWork w{c->ids, c->stage, c->tp_a, nullptr, nullptr};
-    if (text_proj_tiled(c, n)) {
+    w.few = text_proj_few(c, n);
+    if (w.few && ensure_rows(c)) return -1;
+    if (w.few || text_proj_tiled(c, n)) {
         if (n > c->bp_rows) {
             for (void * p : {(void *) c->bp_q, (void *) c->bp_dx, (void *) c->bp_h}) dev_free(c, p);
             c->bp_q = nullptr; c->bp_dx = nullptr; c->bp_h = nullptr; c->bp_rows = 0;
-            if (dev_alloc_t(c, &c->bp_q, (size_t) n * te) || dev_alloc_t(c, &c->bp_dx, (size_t) n * (te / kQK)) ||
-                dev_alloc_t(c, &c->bp_h, (size_t) n * te))
+            const int cap = std::max(n, kRowsMax);
+            if (dev_alloc_t(c, &c->bp_q, (size_t) cap * te) || dev_alloc_t(c, &c->bp_dx, (size_t) cap * (te / kQK)) ||
+                dev_alloc_t(c, &c->bp_h, (size_t) cap * te))
                 return -1;
-            c->bp_rows = n;
+            c->bp_rows = cap;
         }
         w.h = c->bp_h; w.q = c->bp_q; w.dx = c->bp_dx;
     }
@@ -2053,7 +2335,8 @@ int build_rows(q3t_dev * c, const std::vector<int32_t> & ids, const std::vector<
                               hipMemcpyDeviceToHost, c->stream));
     HIP_OK(hipMemcpyAsync(pad_out, c->bp_out + (size_t) (n_pre + n_trail) * d, (size_t) d * 4, hipMemcpyDeviceToHost,
                           c->stream));
-    return sync(c);
+    if (sync(c)) return -1;
+    return rows_check(c);
 }
 
 }  // namespace
@@ -2078,15 +2361,18 @@ int q3t_dev_prefill(q3t_dev * c, const float * embd, int32_t n, int32_t n_past, 
     FrameState s{};
     if (set_state(c, s)) return -1;
     HIP_OK(hipMemcpyAsync(c->stage, embd, (size_t) n * d * 4, hipMemcpyHostToDevice, c->stream));
-    if (const int tp = tiled_prefill(c, n)) {
-        if (ensure_pf(c, n)) return -1;
-        if (tp == 1 ? prefill_mfma(c, n, n_past) : prefill_f16(c, n, n_past)) return -1;
+    const bool rows = rows_prefill(c, n, n_past);
+    if (const int tp = rows ? 3 : tiled_prefill(c, n)) {
+        if (ensure_pf(c, rows ? kRowsMax : n) || (rows && ensure_rows(c))) return -1;
+        if (tp == 3 ? prefill_rows(c, n, n_past) : tp == 1 ? prefill_mfma(c, n, n_past) : prefill_f16(c, n, n_past))
+            return -1;
         if (hidden_out)
             hipLaunchKernelGGL(k_rmsnorm_rows, dim3(n), dim3(kBlock), 0, c->stream, (const float *) c->pf_xa,
                                (const float *) c->out_norm.data, g.rms_eps, d, c->hidden_all);
         if (hidden_out) HIP_OK(hipMemcpyAsync(hidden_out, c->hidden_all, (size_t) n * d * 4, hipMemcpyDeviceToHost, c->stream));
         if (logits_out) HIP_OK(hipMemcpyAsync(logits_out, c->logits, (size_t) g.codec_vocab * 4, hipMemcpyDeviceToHost, c->stream));
-        return sync(c);
+        if (sync(c)) return -1;
+        return rows ? rows_check(c) : 0;
     }
     for (int t0 = 0; t0 < n;) {
         const int left = n - t0;
@@ -2251,7 +2537,8 @@ int q3t_dev_text_proj(q3t_dev * c, const int32_t * tokens, int32_t n, float * ou
     if (ensure_build(c, n, 0, 0)) return -1;
     if (project_rows(c, tokens, n, c->bp_proj)) return -1;
     HIP_OK(hipMemcpyAsync(out, c->bp_proj, (size_t) n * g.hidden_size * 4, hipMemcpyDeviceToHost, c->stream));
-    return sync(c);
+    if (sync(c)) return -1;
+    return rows_check(c);
 }
 
 int q3t_dev_text_proj_noalloc(q3t_dev * c, const int32_t * tokens, int32_t n, float * out) {
@@ -2630,70 +2917,11 @@ struct StreamKV {
     bool f32_prefill;               // the code predictor's 2-token prefill: F32 q, K, V, P
 };
 
-// The three shapes of decode GEMM a layer needs (ms::k_gemm_sk):
-//   QKV      RMSNorm'd fp32 rows quantised in registers, fp32 out
-//   PROJ     pre-quantised rows in (attention / SwiGLU output), + residual
-//   GATE_UP  RMSNorm'd rows, gate and up matrices, SwiGLU, Q8_0 out
-enum GemmKind { G_QKV = 0, G_PROJ = 1, G_GATE_UP = 2 };
-// preferred K splits and the Q8_0 blocks per wave they leave (QKV and gate/up:
-// 32 blocks / (4 waves x 2); Wo / down: 64 or 96 / (4 x 4)).  Measured with
-// 16 streams on one box: {2, 4, 2} 2,567 aggregate frames/s, {2, 2, 2} 2,500,
-// the former {4, 8, 4} 2,340, no split {1, 1, 1} 2,051.
-constexpr int kGemmKB[3] = {4, 6, 4};       // max Q8_0 blocks per wave
-constexpr int kGemmMT[3] = {1, 1, 2};       // 16-row tiles per workgroup
-constexpr int kGemmS[3] = {2, 4, 2};        // preferred K splits
-
-template <int NT, int KIND>
-const void * gemm_kernel() {
-    if (KIND == G_QKV) return (const void *) ms::k_gemm_sk<NT, 1, false, ms::IN_NORM, ms::OUT_F32, kGemmKB[G_QKV]>;
-    if (KIND == G_PROJ) return (const void *) ms::k_gemm_sk<NT, 1, false, ms::IN_Q8, ms::OUT_RESID, kGemmKB[G_PROJ]>;
-    return (const void *) ms::k_gemm_sk<NT, 2, true, ms::IN_NORM, ms::OUT_SWIGLU_Q8, kGemmKB[G_GATE_UP]>;
-}
-
-template <int KIND>
-const void * gemm_kernel_nt(int nt) {
-    switch (nt) {
-        case 1: return gemm_kernel<1, KIND>();
-        case 2: return gemm_kernel<2, KIND>();
-        case 3: return gemm_kernel<3, KIND>();
-        default: return gemm_kernel<4, KIND>();
-    }
-}
-
-const void * gemm_fn(int kind, int nt) {
-    return kind == G_QKV ? gemm_kernel_nt<G_QKV>(nt) : kind == G_PROJ ? gemm_kernel_nt<G_PROJ>(nt)
-                                                                      : gemm_kernel_nt<G_GATE_UP>(nt);
-}
-
-// K splits for a contraction of nb Q8_0 blocks: the largest S <= the kind's
-// preference with nb % (4 S) == 0 and at most KB blocks per wave; 0 if none.
-int gemm_splits(int kind, int nb) {
-    for (int S = kGemmS[kind]; S >= 1; S >>= 1)
-        if (nb % (ms::kWaves * S) == 0 && nb / (ms::kWaves * S) <= kGemmKB[kind]) return S;
-    return 0;
-}
-
-size_t gemm_lds(int kind, int nt, int K) {
-    const int S = gemm_splits(kind, K / kQK);
-    return ms::gemm_sk_lds_bytes(nt, kGemmMT[kind], kind == G_GATE_UP, S ? K / kQK / S : 0);
-}
-
-// tagged words of the partials one launch may store: tiles x S x 2 per value x values per lane x 64 lanes
-size_t gemm_part_words(int kind, int nt, int N, int K) {
-    const int mt = kGemmMT[kind], nw = kind == G_GATE_UP ? 2 : 1;
-    return (size_t) (N / (ms::kRows * mt)) * gemm_splits(kind, K / kQK) * 2 * nw * mt * nt * 4 * 64;
-}
-
 // call types sharing a ticket/partial set
 enum GemmSite { S_QKV = 0, S_WO = 1, S_GATE_UP = 2, S_DOWN = 3 };
 
-void gemm_rows(q3t_dev * c, int kind, int site, ms::GemmArgs a) {
-    const int nt = (a.n + 15) / 16;
-    const int S = gemm_splits(kind, a.K / kQK);
-    a.part = c->spart[site]; a.cnt = c->scnt[site]; a.err = c->serr;
-    void * args[] = {(void *) &a};
-    (void) hipLaunchKernel(gemm_fn(kind, nt), dim3(a.N / (ms::kRows * kGemmMT[kind]), S), dim3(ms::kThreads), args,
-                           gemm_lds(kind, nt, a.K), c->stream);
+void gemm_rows(q3t_dev * c, int kind, int site, const ms::GemmArgs & a) {
+    gemm_sk(c, kind, a, c->spart[site], c->scnt[site], c->serr);
 }
 
 // F16 layers: the four decode GEMMs of a layer on ms::k_gemm_h, 16-row tiles,
@@ -2768,22 +2996,6 @@ void hgemm_rows(q3t_dev * c, int kind, int site, ms::GemmArgs a) {
 // Contraction length of each decode GEMM kind: the normed inputs are model
 // rows (d), the projections read attention or SwiGLU rows.
 int gemm_k(int kind, int d, int kproj) { return kind == G_PROJ ? kproj : d; }
-
-// Allows each decode GEMM its dynamic LDS.
-hipError_t allow_gemm_lds(int d, int kproj) {
-    for (int kind = 0; kind < 3; ++kind)
-        for (int nt = 1; nt <= 4; ++nt) {
-            const hipError_t e = hipFuncSetAttribute(gemm_fn(kind, nt), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                     (int) gemm_lds(kind, nt, gemm_k(kind, d, kproj)));
-            if (e != hipSuccess) return e;
-        }
-    return hipSuccess;
-}
-
-// RMSNorm row scales of n rows of width K into c->srs.
-void row_scales(q3t_dev * c, const float * x, int xs, int K, int n) {
-    hipLaunchKernelGGL(ms::k_row_scale, dim3(n), dim3(kBlock), 0, c->stream, x, xs, K, c->cfg.rms_eps, c->srs);
-}
 
 void attn_gqa(q3t_dev * c, const LayerDev & L, const StreamKV & kv) {
     const q3t_config & g = c->cfg;
@@ -2875,7 +3087,7 @@ static void stream_layer(q3t_dev * c, const LayerDev & L, const float * x, bool 
     if (tab_step > 0) {
         cp_tab_rows(c, tab_step);
     } else {
-        if (!x_ss) row_scales(c, x, d, d, n);
+        if (!x_ss) row_scales(c, x, d, d, n, c->srs);
         ms::GemmArgs q{};
         q.W = (const int8_t *) L.qkv.data; q.Wd = L.qkv.scales; q.N = qkvd; q.K = d;
         q.x = x; q.xs = d; q.rscale = c->srs; q.norm_w = L.attn_norm; q.n = n; q.y = c->bqkv; q.ys = qkvd;
@@ -2888,7 +3100,7 @@ static void stream_layer(q3t_dev * c, const LayerDev & L, const float * x, bool 
     o.q = c->bq8; o.qdx = c->bdx8; o.n = n; o.y = c->bxb; o.ys = d; o.res = x; o.rs = d;
     if (fuse) o.ss_out = c->sss[0];
     gemm_rows(c, G_PROJ, S_WO, o);
-    if (!fuse) row_scales(c, c->bxb, d, d, n);
+    if (!fuse) row_scales(c, c->bxb, d, d, n, c->srs);
     ms::GemmArgs f{};
     f.W = (const int8_t *) L.wg.data; f.Wd = L.wg.scales; f.W2 = (const int8_t *) L.wu.data; f.W2d = L.wu.scales;
     f.N = ffn; f.K = d; f.x = c->bxb; f.xs = d; f.rscale = c->srs; f.norm_w = L.ffn_norm; f.n = n;
@@ -2915,7 +3127,7 @@ static void stream_layer_h(q3t_dev * c, const LayerDev & L, const float * x, boo
     if (tab_step > 0) {
         cp_tab_rows(c, tab_step);
     } else {
-        if (!x_ss) row_scales(c, x, d, d, n);
+        if (!x_ss) row_scales(c, x, d, d, n, c->srs);
         ms::GemmArgs q{};
         q.H = (const uint16_t *) L.qkv.data; q.N = qkvd; q.K = d;
         q.x = x; q.xs = d; q.rscale = c->srs; q.norm_w = L.attn_norm; q.n = n; q.y = c->bqkv; q.ys = qkvd;
@@ -2928,7 +3140,7 @@ static void stream_layer_h(q3t_dev * c, const LayerDev & L, const float * x, boo
     o.x = c->batt; o.xs = qd; o.n = n; o.y = c->bxb; o.ys = d; o.res = x; o.rs = d;
     if (fuse) o.ss_out = c->sss[0];
     hgemm_rows(c, H_WO, S_WO, o);
-    if (!fuse) row_scales(c, c->bxb, d, d, n);
+    if (!fuse) row_scales(c, c->bxb, d, d, n, c->srs);
     ms::GemmArgs f{};
     f.H = (const uint16_t *) L.wg.data; f.H2 = (const uint16_t *) L.wu.data; f.N = ffn; f.K = d;
     f.x = c->bxb; f.xs = d; f.rscale = c->srs; f.norm_w = L.ffn_norm; f.n = n; f.y = c->bff; f.ys = ffn;
@@ -3032,8 +3244,9 @@ int q3t_dev_streams_reserve(q3t_dev * c, int32_t n_streams, int32_t n_ctx) {
     const int G = g.n_kv_head > 0 ? g.n_head / g.n_kv_head : 0;
     // decode GEMMs: every contraction splits into 4-wave slices of at most KB
     // blocks (32-element chunks) per wave; N a multiple of 16 (Q8_0 gate/up: 32)
-    const bool splits_ok = all_q8 ? gemm_splits(G_QKV, d / kQK) && gemm_splits(G_GATE_UP, d / kQK) &&
-                                        gemm_splits(G_PROJ, qd / kQK) && gemm_splits(G_PROJ, g.ffn_size / kQK)
+    const auto q8_ok = [](int kind, int nb) { const int S = gemm_splits(kind, nb); return S > 0 && S <= kGemmS[kind]; };
+    const bool splits_ok = all_q8 ? q8_ok(G_QKV, d / kQK) && q8_ok(G_GATE_UP, d / kQK) && q8_ok(G_PROJ, qd / kQK) &&
+                                        q8_ok(G_PROJ, g.ffn_size / kQK)
                                   : hgemm_splits(H_QKV, d / kQK) && hgemm_splits(H_GATE_UP, d / kQK) &&
                                         hgemm_splits(H_WO, qd / kQK) && hgemm_splits(H_DOWN, g.ffn_size / kQK);
     if (g.head_dim != 128 || d % kQK || qd % kQK || g.ffn_size % kQK || !splits_ok || qkvd % ms::kRows ||
@@ -3048,7 +3261,7 @@ int q3t_dev_streams_reserve(q3t_dev * c, int32_t n_streams, int32_t n_ctx) {
     for (int kind = 0; kind < 3; ++kind) gl = std::max(gl, gemm_lds(kind, 4, gemm_k(kind, d, kproj)));
     if (gl > (size_t) max_lds) return fail(c, "multi-stream decode: GEMM LDS exceeds the device limit");
     if (al > (size_t) max_lds) return fail(c, "multi-stream decode: n_ctx too large for the attention kernel's LDS");
-    HIP_OK(allow_gemm_lds(d, kproj));
+    HIP_OK(allow_gemm_lds(max_lds));
     HIP_OK(hipFuncSetAttribute((const void *) ms::k_attn_gqa<1>, hipFuncAttributeMaxDynamicSharedMemorySize, (int) al));
     // the streams' talker caches share the context's RoPE tables and KV layout stride
     if (c->n_ctx != n_ctx && q3t_dev_kv_reserve(c, n_ctx)) return -1;

@@ -42,8 +42,8 @@ constexpr int kWaves = 4;             // waves per workgroup, each a part of the
 constexpr int kThreads = kWaves * 64;
 constexpr int kMaxTok = 64;           // activation rows per launch (4 MFMA column tiles)
 
-enum GemmIn { IN_Q8 = 0, IN_NORM = 1, IN_ROUND = 2, IN_WIDE = 3 };
-enum GemmOut { OUT_F32 = 0, OUT_RESID = 1, OUT_SWIGLU_Q8 = 2, OUT_SWIGLU_F32 = 3 };
+enum GemmIn { IN_Q8 = 0, IN_NORM = 1, IN_ROUND = 2, IN_WIDE = 3, IN_PLAIN = 4 };
+enum GemmOut { OUT_F32 = 0, OUT_RESID = 1, OUT_SWIGLU_Q8 = 2, OUT_SWIGLU_F32 = 3, OUT_BIAS_SILU = 4 };
 
 struct GemmArgs {
     const int8_t * W; const uint16_t * Wd;     // [N][K] int8, [N][K/32] fp16 scales
@@ -51,23 +51,23 @@ struct GemmArgs {
     const uint16_t * H; const uint16_t * H2;   // F16 weights [N][K] (k_gemm_h; H2: the up matrix)
     int32_t N, K;
     const int8_t * q; const float * qdx;       // IN_Q8: activation rows [n][K] int8, scales [n][K/32]
-    const float * x; int32_t xs;               // IN_NORM: activation rows [n][xs] fp32
+    const float * x; int32_t xs;               // IN_NORM, IN_PLAIN: activation rows [n][xs] fp32
     const float * rscale;                      //          1/sqrt(mean(x^2) + eps) per row, or:
     const double * ss_in; int32_t ss_tiles;    //          the producing GEMM's per-tile sums of squares [tiles][n]
     float eps;
     const float * norm_w;                      //          RMSNorm gain [K]
     int32_t n;                                 // activation rows, <= 16 * NT
     float * y; int32_t ys;                     // OUT_F32 / OUT_RESID rows [n][ys]
-    const float * res; int32_t rs;             // OUT_RESID residual rows [n][rs]
+    const float * res; int32_t rs;             // OUT_RESID residual rows [n][rs] (rs = 0: one bias row)
     double * ss_out;                           // OUT_RESID: per-tile sums of squares of the rows [tiles][n] (or NULL)
     int8_t * yq; float * ydx;                  // OUT_SWIGLU_Q8 rows [n][N] int8, scales [n][N/32]
     uint64_t * part;                           // split-K partials [tiles][S][2 NV][64] tagged words
     uint32_t * cnt;                            // per-tile arrival counters (S per launch, never reset)
-    int32_t * err;                             // set when a split-K wait times out
+    int32_t * err;                             // set when a split-K wait times out (device or mapped host memory)
 };
 
 constexpr unsigned kSkSpin = 1u << 20;     // polls before a split-K wait gives up
-constexpr int kSsPer = 16;                 // per-tile sums of squares one lane adds (hidden <= 1024)
+constexpr int kSsPer = 16;                 // per-tile sums of squares one lane has in flight
 
 // Dynamic LDS: weight scales of the slice [NW][MT*16][K/32/S] f32 and the
 // cross-wave partials [2][NW][MT][NT][4][64] f64.
@@ -164,7 +164,11 @@ __device__ __forceinline__ bool splitk_exchange(double (&acc)[NV], const GemmArg
 #pragma unroll
                 for (int k = 0; k < 2 * CH; ++k) all = all && (uint32_t) (w[k] >> 32) == tag;
                 if (__all(all)) break;
-                if (++n > kSkSpin) { dead = true; atomicExch(a.err, 1); break; }
+                if (++n > kSkSpin) {
+                    dead = true;
+                    __hip_atomic_store(a.err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+                    break;
+                }
                 __builtin_amdgcn_s_sleep(1);
 #pragma unroll
                 for (int k = 0; k < 2 * CH; ++k)
@@ -203,6 +207,7 @@ template <int NT, int MT, bool DUAL, int IN, int OUT, int KB>
 __global__ __launch_bounds__(kThreads) void k_gemm_sk(GemmArgs a) {
     constexpr int NW = DUAL ? 2 : 1;
     constexpr bool QIN = IN == IN_Q8;
+    constexpr bool ADD = OUT == OUT_RESID || OUT == OUT_BIAS_SILU;
     constexpr int NV = NW * MT * NT * 4;             // fp64 partials per lane
     extern __shared__ __align__(16) char smem[];
     const int nb = a.K / kQK, S = gridDim.y, nbs = nb / S, bpw = nbs / kWaves;
@@ -245,18 +250,22 @@ __global__ __launch_bounds__(kThreads) void k_gemm_sk(GemmArgs a) {
                 }
         } else {
             const float * xr = a.x + (size_t) (ok ? tok : 0) * a.xs + 8 * lk;
-            if (a.ss_in) {
+            if (IN == IN_PLAIN) {
+                rsc[QIN ? 0 : j] = 0.0f;                  // not used
+            } else if (a.ss_in) {
                 // RMSNorm row scale from the producer's per-tile sums: lane
                 // group lk adds a quarter of the tiles in order, then a fixed
                 // pairwise tree ((q0 + q1) + (q2 + q3))
-                const int per = a.ss_tiles / 4;   // <= kSsPer (the host checks)
-                double sv[kSsPer];
-#pragma unroll
-                for (int i = 0; i < kSsPer; ++i)
-                    sv[i] = ok && i < per ? a.ss_in[(size_t) (lk * per + i) * a.n + tok] : 0.0;
+                const int per = a.ss_tiles / 4;
                 double part = 0.0;
+                for (int i0 = 0; i0 < per; i0 += kSsPer) {
+                    double sv[kSsPer];
 #pragma unroll
-                for (int i = 0; i < kSsPer; ++i) part += sv[i];
+                    for (int i = 0; i < kSsPer; ++i)
+                        sv[i] = ok && i0 + i < per ? a.ss_in[(size_t) (lk * per + i0 + i) * a.n + tok] : 0.0;
+#pragma unroll
+                    for (int i = 0; i < kSsPer; ++i) part += sv[i];
+                }
                 part += __shfl_xor(part, 16);
                 part += __shfl_xor(part, 32);
                 const float mean = (float) (part / (double) a.K);
@@ -276,11 +285,11 @@ __global__ __launch_bounds__(kThreads) void k_gemm_sk(GemmArgs a) {
             }
         }
     }
-    // OUT_RESID: wave 0 runs the epilogue if this workgroup arrives last; its
+    // OUT_RESID (a bias too): wave 0 runs the epilogue if this workgroup arrives last; its
     // residual values are loaded now, so the epilogue does not wait on them
     // (no workgroup writes the tile's rows before the last arriver)
-    float rres[OUT == OUT_RESID ? NT : 1][OUT == OUT_RESID ? MT : 1][4];
-    if constexpr (OUT == OUT_RESID) {
+    float rres[ADD ? NT : 1][ADD ? MT : 1][4];
+    if constexpr (ADD) {
         if (wave == 0) {
 #pragma unroll
             for (int j = 0; j < NT; ++j) {
@@ -317,15 +326,16 @@ __global__ __launch_bounds__(kThreads) void k_gemm_sk(GemmArgs a) {
                 bop = qb[j][i];
                 dxv = qd[j][i];
             } else {
-                // RMSNorm y = (x * scale) * w, then Q8_0 of the block
-                const float * nw = a.norm_w + b * kQK + 8 * lk;
-                const float4 g0 = *(const float4 *) nw, g1 = *(const float4 *) (nw + 4);
+                // RMSNorm y = (x * scale) * w (IN_PLAIN: x), then Q8_0 of the block
                 const float4 u0 = xv[QIN ? 0 : j][QIN ? 0 : i][0], u1 = xv[QIN ? 0 : j][QIN ? 0 : i][1];
-                const float xs8[8] = {u0.x, u0.y, u0.z, u0.w, u1.x, u1.y, u1.z, u1.w};
-                const float gs8[8] = {g0.x, g0.y, g0.z, g0.w, g1.x, g1.y, g1.z, g1.w};
-                float v[8];
+                float v[8] = {u0.x, u0.y, u0.z, u0.w, u1.x, u1.y, u1.z, u1.w};
+                if (IN == IN_NORM) {
+                    const float * nw = a.norm_w + b * kQK + 8 * lk;
+                    const float4 g0 = *(const float4 *) nw, g1 = *(const float4 *) (nw + 4);
+                    const float gs8[8] = {g0.x, g0.y, g0.z, g0.w, g1.x, g1.y, g1.z, g1.w};
 #pragma unroll
-                for (int e = 0; e < 8; ++e) { const float sv = xs8[e] * rsc[QIN ? 0 : j]; v[e] = sv * gs8[e]; }
+                    for (int e = 0; e < 8; ++e) { const float sv = v[e] * rsc[QIN ? 0 : j]; v[e] = sv * gs8[e]; }
+                }
                 bop = quant8(v, dxv);
             }
 #pragma unroll
@@ -412,8 +422,9 @@ __global__ __launch_bounds__(kThreads) void k_gemm_sk(GemmArgs a) {
                 for (int e = 0; e < 4; ++e) {
                     const float v = (float) acc[(m * NT + j) * 4 + e];
                     float rv = 0.0f;
-                    if constexpr (OUT == OUT_RESID) rv = rres[j][m][e];
-                    o[e] = OUT == OUT_RESID && ok ? v + rv : v;
+                    if constexpr (ADD) rv = rres[j][m][e];
+                    o[e] = ADD && ok ? v + rv : v;
+                    if (OUT == OUT_BIAS_SILU) o[e] = silu_q3t(o[e]);
                     sq += (double) (o[e] * o[e]);
                 }
                 if (ok) *(float4 *) (a.y + (size_t) tok * a.ys + r0 + 16 * m + 4 * lk) = make_float4(o[0], o[1], o[2], o[3]);
@@ -694,8 +705,9 @@ struct GqaArgs {
     uint16_t * kc; uint16_t * vc;              // layer base of stream 0, [n_kv_head][n_ctx][128]
     int64_t kv_stream;                         // elements per stream
     int32_t n_ctx, n_head, n_kv_head;
-    const int32_t * pos; int32_t pos_stream;   // position of stream s at pos[s * pos_stream] (NULL: pos_const)
-    int32_t pos_const;
+    const int32_t * pos; int32_t pos_stream;   // position of stream s at pos[s * pos_stream], or (pos NULL)
+    int32_t pos_const, pos_row;                //   at pos_const + s * pos_row
+    int32_t no_append;                         // the new rows are in the cache already (rows of one prefill)
     const int32_t * done; int32_t done_stream; // stream s idles while done[s * done_stream] (NULL: never)
     float * out; int32_t out_stride;           // stream s's [n_head * 128] row
     int8_t * out_q; float * out_dx;            // its Q8_0 copy: [n_head * 128] int8, [n_head * 4] scales (NULL: none)
@@ -713,13 +725,15 @@ __host__ __device__ constexpr size_t attn_gqa_lds_bytes(int g, int n_ctx) {
 // Workgroup x takes query heads G x .. G x + G - 1 of stream blockIdx.y; with
 // G below the group size two or more workgroups share a KV head, read its
 // cache each, and only the first appends the new K/V row (the others take
-// the new row from their own LDS).  BF: a bfloat16 cache (q and P rounded to
+// the new row from their own LDS).  The rows of one prefill are "streams" of
+// one cache (kv_stream 0) at consecutive positions, all appended before the
+// launch (no_append).  BF: a bfloat16 cache (q and P rounded to
 // bfloat16 as well).
 template <int G, bool BF = false>
 __global__ __launch_bounds__(kAThreads) void k_attn_gqa(GqaArgs a) {
     const int hq0 = blockIdx.x * G, z = blockIdx.y;
     const int gsz = a.n_head / a.n_kv_head, g = hq0 / gsz;
-    const bool append = hq0 % gsz == 0;
+    const bool append = hq0 % gsz == 0 && !a.no_append;
     if (a.done && a.done[(size_t) z * a.done_stream]) return;
     extern __shared__ __align__(16) char smem[];
     float * qf = (float *) smem;                  // [G][128] fp16-rounded rotated q
@@ -731,7 +745,7 @@ __global__ __launch_bounds__(kAThreads) void k_attn_gqa(GqaArgs a) {
     double * pv = (double *) sc;                  // after the scores are consumed: [16][G][128]
 
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    const int pos = a.pos ? a.pos[(size_t) z * a.pos_stream] : a.pos_const, n_kv = pos + 1;
+    const int pos = a.pos ? a.pos[(size_t) z * a.pos_stream] : a.pos_const + z * a.pos_row, n_kv = pos + 1;
     const int qd = a.n_head * kHD, kd = a.n_kv_head * kHD;
     const float * row = a.qkv + (size_t) z * a.qkv_stride;
     uint16_t * kbase = a.kc + z * a.kv_stream + (size_t) g * a.n_ctx * kHD;
