@@ -490,6 +490,38 @@ int st_input_proj(q3t_voc * v, int64_t n, const Io & io) {
                 v->xf, H, nullptr, 0, ACT_NONE, nullptr);
 }
 
+constexpr size_t kAttnTileLds = (size_t) 144 << 10;
+
+template <int HD, int R>
+void attn_tiled(q3t_voc * v, int64_t n, int32_t L, int32_t Q, float asc) {
+    hipLaunchKernelGGL((k_attn_causal_tile<HD, R>), dim3((unsigned) ((n + 4 * R - 1) / (4 * R)), (unsigned) v->cfg.n_heads),
+                       dim3(256), attn_tile_lds_bytes(HD, 4 * R, (int) n), v->stream, v->qkv, Q, v->cfg.latent,
+                       (int32_t) n, asc, v->att, L);
+}
+
+// Causal attention over the n qkv rows into v->att.  Head widths 32 and 64:
+// 64-key tiles in LDS while a workgroup's scores fit (7,900 frames with one
+// query row per wave), two rows per wave above 64 frames (whole decodes, one /
+// two / four rows a wave: 64 frames 1,670 / 1,668 / 1,731 us, 73 1,837 / 1,817 /
+// 1,880, 600 10,159 / 10,095 / 10,150); other widths and longer decodes the
+// one-wave-per-row kernel (73 frames 1,917, 241 frames 5,232 against 4,287, 600
+// frames 15,497).  All forms give the same bits, so a decode stays the prefix
+// of a longer one.
+int attn_causal(q3t_voc * v, int64_t n, int32_t hd, int32_t L, int32_t Q) {
+    const float asc = 1.0f / std::sqrt((float) hd);
+    const auto fits = [&](int R) { return attn_tile_lds_bytes(hd, 4 * R, (int) n) <= kAttnTileLds; };
+    const int R = hd != 32 && hd != 64 ? 0 : n > 64 && fits(2) ? 2 : fits(1) ? 1 : 0;
+    if (R == 2 && hd == 64) attn_tiled<64, 2>(v, n, L, Q, asc);
+    else if (R == 1 && hd == 64) attn_tiled<64, 1>(v, n, L, Q, asc);
+    else if (R == 2) attn_tiled<32, 2>(v, n, L, Q, asc);
+    else if (R == 1) attn_tiled<32, 1>(v, n, L, Q, asc);
+    else
+        hipLaunchKernelGGL(k_attn_causal, dim3((unsigned) n, (unsigned) v->cfg.n_heads), dim3(64), (size_t) n * 4,
+                           v->stream, v->qkv, Q, v->cfg.latent, hd, asc, v->att, L);
+    HIP_OK(hipGetLastError());
+    return 0;
+}
+
 int st_pre_tfm(q3t_voc * v, int l, int64_t n, int32_t pos0) {
     const q3t_voc_config & c = v->cfg;
     const PreLayer & P = v->pre[(size_t) l];
@@ -505,22 +537,7 @@ int st_pre_tfm(q3t_voc * v, int l, int64_t n, int32_t pos0) {
     hipLaunchKernelGGL(k_rope_qk, dim3((unsigned) ((nr + 255) / 256)), dim3(256), 0, v->stream, v->qkv, Q, (int32_t) n,
                        c.latent, hd, v->rope_cos, v->rope_sin, pos0);
     HIP_OK(hipGetLastError());
-    // windows whose K and V rows fit in LDS take the staged kernel (4 query
-    // rows per workgroup, head widths 32 and 64); longer decodes the
-    // one-wave-per-row kernel
-    const size_t lds = ((size_t) 2 * n * hd + (size_t) 4 * hd + (size_t) 4 * n) * 4;
-    const dim3 sg((unsigned) ((n + 3) / 4), (unsigned) c.n_heads);
-    const float asc = 1.0f / std::sqrt((float) hd);
-    if (lds <= 65536 && hd == 64)
-        hipLaunchKernelGGL(k_attn_causal_lds<64>, sg, dim3(256), lds, v->stream, v->qkv, Q, c.latent, (int32_t) n, asc,
-                           v->att, L);
-    else if (lds <= 65536 && hd == 32)
-        hipLaunchKernelGGL(k_attn_causal_lds<32>, sg, dim3(256), lds, v->stream, v->qkv, Q, c.latent, (int32_t) n, asc,
-                           v->att, L);
-    else
-        hipLaunchKernelGGL(k_attn_causal, dim3((unsigned) n, (unsigned) c.n_heads), dim3(64), (size_t) n * 4, v->stream,
-                           v->qkv, Q, c.latent, hd, 1.0f / std::sqrt((float) hd), v->att, L);
-    HIP_OK(hipGetLastError());
+    if (attn_causal(v, n, hd, L, Q)) return -1;
     if (gemm(v, P.wo, v->att, L, (int32_t) n, 0, 1, (int32_t) n, 1, nullptr, P.attn_scale, v->xf, H, v->xf, H,
              nullptr, 0, ACT_NONE, nullptr))
         return -1;
@@ -745,6 +762,10 @@ q3t_voc * q3t_voc_create(const q3t_voc_config * cfg, int32_t device, const char 
         delete v;
         return bad("hipStreamCreate failed");
     }
+    // the tiled attention's scores may take more LDS than the 64 KiB default
+    for (const void * f : {(const void *) k_attn_causal_tile<64, 1>, (const void *) k_attn_causal_tile<64, 2>,
+                           (const void *) k_attn_causal_tile<32, 1>, (const void *) k_attn_causal_tile<32, 2>})
+        (void) hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int) kAttnTileLds);
     if (alloc(v, &v->bad, 1)) {
         last = v->err;
         q3t_voc_destroy(v);

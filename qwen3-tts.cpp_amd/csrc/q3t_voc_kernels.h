@@ -664,82 +664,145 @@ __global__ __launch_bounds__(64) void k_attn_causal(const float * __restrict__ q
     }
 }
 
-// k_attn_causal for short windows: workgroup (x, h) takes query rows 4x ..
-// 4x + 3 of head h, one wave each, with their q rows and the head's K and V
-// rows 0 .. 4x + 3 staged in LDS once, and the head width a constant so the
-// dot products unroll (the one-wave kernel reads q, K and V from global
-// memory inside its dependent fp64 chains).  Every lane computes what it
-// computes there, in the same order: scores as sequential fp64 fmas over
-// the head dims, the max and fp64 sum over the same lane split and shuffle
-// tree, P.V as one dim per lane over the keys in order.  Dynamic LDS:
-// (2 T HD + 4 HD + 4 T) floats.
-template <int HD>
-__global__ __launch_bounds__(256) void k_attn_causal_lds(const float * __restrict__ qkv, int32_t qs, int32_t L, int32_t T,
-                                                         float scale, uint16_t * __restrict__ out, int32_t os) {
-    extern __shared__ float sm[];
+// k_attn_causal for any length that a workgroup's scores fit: workgroup (x, h)
+// takes query rows 4R x .. 4R x + 4R - 1 of head h, R per wave, and streams the
+// head's K and then V rows through one 64-key LDS tile (the next tile's loads
+// in flight meanwhile), so a key row is read once for 4R queries and no wave
+// waits on global memory inside its dependent fp64 chains; the R rows of a wave
+// are R independent chains.  241 frames: 138 us a launch with one wave per row
+// reading q, K and V from global memory, 14 here.  The arithmetic and its order are k_attn_causal's:
+// scores as sequential fp64 fmas over the head dims, the maximum and the fp64
+// sum over the same lane split (key mod 64) and shuffle tree, P.V as one dim per
+// lane over the keys in order.  Keys past a row's own are never accumulated.
+// Dynamic LDS: tile 64 (HD + 1) floats, q 4R x HD doubles, scores 4R x ts
+// floats (ts = T rounded up to 64).
+__host__ __device__ constexpr size_t attn_tile_lds_bytes(int hd, int rows, int T) {
+    return (size_t) 64 * (hd + 1) * 4 + (size_t) rows * hd * 8 + (size_t) rows * ((T + 63) / 64 * 64) * 4;
+}
+template <int HD, int R>
+__global__ __launch_bounds__(256) void k_attn_causal_tile(const float * __restrict__ qkv, int32_t qs, int32_t L, int32_t T,
+                                                          float scale, uint16_t * __restrict__ out, int32_t os) {
+    extern __shared__ __align__(16) char smem[];
+    constexpr int KS = HD + 1;                        // K tile [d][key] has stride 65; V tile [key][d] stride HD
+    constexpr int NL = 64 * HD / 4 / 256;             // float4 loads per thread and tile
+    static_assert(HD <= 64 && 64 * HD % 1024 == 0, "head width");
+    double * qd = (double *) smem;                    // [4R][HD]
+    float * tile = (float *) (qd + 4 * R * HD);
+    float * sc = tile + 64 * KS;
+    const int ts = (T + 63) / 64 * 64;
     const int h = blockIdx.y, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int t0 = blockIdx.x * 4, t = t0 + wave;
-    const int nrow = min(t0 + 4, T);                  // keys 0 .. nrow - 1 cover every row of the workgroup
-    // K transposed ([d][key], stride T), so the lanes of a wave, one key
-    // each, read consecutive words; V as rows ([key][d]), read one dim per lane
-    float * ks = sm;                                  // [HD][T]
-    float * vs = sm + (size_t) T * HD;                // [nrow][HD]
-    float * qv = sm + (size_t) 2 * T * HD;            // [4][HD]
-    float * p = qv + 4 * HD + (size_t) wave * T;      // [T] per wave
-    // 8 elements of K and of V per thread in flight before they are stored
-    constexpr int U = 8;
-    for (int i0 = threadIdx.x; i0 < nrow * HD; i0 += 256 * U) {
-        float kv[U], vv[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int i = i0 + 256 * u, j = i / HD, d = i - j * HD;
-            if (i < nrow * HD) {
-                kv[u] = qkv[(size_t) j * qs + L + h * HD + d];
-                vv[u] = qkv[(size_t) j * qs + 2 * L + h * HD + d];
-            }
-        }
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int i = i0 + 256 * u, j = i / HD, d = i - j * HD;
-            if (i < nrow * HD) {
-                ks[(size_t) d * T + j] = kv[u];
-                vs[i] = vv[u];
-            }
-        }
-    }
-    for (int i = threadIdx.x; i < 4 * HD; i += 256) {
+    const int t0 = blockIdx.x * 4 * R, tw = t0 + wave * R;   // this wave's rows: tw .. tw + R - 1
+    const int last = min(t0 + 4 * R, T) - 1;          // last key any row of the workgroup sees
+    float * p = sc + (size_t) wave * R * ts;          // [R][ts]
+    for (int i = threadIdx.x; i < 4 * R * HD; i += 256) {
         const int r = t0 + i / HD;
-        qv[i] = r < T ? qkv[(size_t) r * qs + h * HD + i % HD] : 0.0f;
+        qd[i] = r < T ? (double) qkv[(size_t) r * qs + h * HD + i % HD] : 0.0;
     }
-    __syncthreads();
-    const bool act = t < T;                           // wave-uniform: the last workgroup's spare waves idle
-    float inv = 0.0f;
-    if (act) {
-        const float * q = qv + wave * HD;
-        float mx = -INFINITY;
-        for (int j = lane; j <= t; j += 64) {
-            double s = 0.0;
+    float4 st[NL];
+    auto fetch = [&](int j0, int part) {              // part 1: K, 2: V
 #pragma unroll
-            for (int d = 0; d < HD; ++d) s = fma((double) q[d], (double) ks[(size_t) d * T + j], s);
-            const float v = (float) s * scale;
-            p[j] = v;
-            mx = fmaxf(mx, v);
+        for (int u = 0; u < NL; ++u) {
+            const int i = threadIdx.x + 256 * u, j = j0 + i / (HD / 4), d = (i % (HD / 4)) * 4;
+            st[u] = j <= last ? *(const float4 *) (qkv + (size_t) j * qs + (size_t) part * L + h * HD + d)
+                              : make_float4(0.f, 0.f, 0.f, 0.f);
         }
-        for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
+    };
+    float mx[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) mx[r] = -INFINITY;
+    fetch(0, 1);
+    for (int j0 = 0; j0 <= last; j0 += 64) {
+        __syncthreads();                              // the tile before is used up (first: q staged)
+#pragma unroll
+        for (int u = 0; u < NL; ++u) {
+            const int i = threadIdx.x + 256 * u, j = i / (HD / 4), d = (i % (HD / 4)) * 4;
+            tile[(d + 0) * 65 + j] = st[u].x;
+            tile[(d + 1) * 65 + j] = st[u].y;
+            tile[(d + 2) * 65 + j] = st[u].z;
+            tile[(d + 3) * 65 + j] = st[u].w;
+        }
+        __syncthreads();
+        if (j0 + 64 <= last) fetch(j0 + 64, 1);
+        else fetch(0, 2);                             // the first V tile
+        if (j0 > tw + R - 1) continue;                // past every row of this wave (uniform)
+        double s[R];
+#pragma unroll
+        for (int r = 0; r < R; ++r) s[r] = 0.0;
+#pragma unroll 16
+        for (int d = 0; d < HD; ++d) {
+            const double kd = (double) tile[d * 65 + lane];
+#pragma unroll
+            for (int r = 0; r < R; ++r) s[r] = fma(qd[(wave * R + r) * HD + d], kd, s[r]);
+        }
+        const int j = j0 + lane;
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+            if (j <= tw + r) {
+                const float v = (float) s[r] * scale;
+                p[r * ts + j] = v;
+                mx[r] = fmaxf(mx[r], v);
+            }
+    }
+    // softmax of the wave's rows: each lane reads back the keys it wrote
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const int t = tw + r;
+        if (t >= T) continue;                         // uniform: a spare row of the last workgroup
+        float m = mx[r];
+        for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o));
         double sum = 0.0;
         for (int j = lane; j <= t; j += 64) {
-            const float e = expf(p[j] - mx);
-            p[j] = e;
+            const float e = expf(p[r * ts + j] - m);
+            p[r * ts + j] = e;
             sum += (double) e;
         }
         for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o);
-        inv = (float) (1.0 / sum);
+        const float inv = (float) (1.0 / sum);
+        for (int j = lane; j <= t; j += 64) p[r * ts + j] = p[r * ts + j] * inv;
     }
-    __syncthreads();
-    if (act && lane < HD) {
-        double o = 0.0;
-        for (int j = 0; j <= t; ++j) o = fma((double) (p[j] * inv), (double) vs[(size_t) j * HD + lane], o);
-        out[(size_t) t * os + h * HD + lane] = f2h((float) o);
+    double o[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) o[r] = 0.0;
+    for (int j0 = 0; j0 <= last; j0 += 64) {
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < NL; ++u) {
+            const int i = threadIdx.x + 256 * u, j = i / (HD / 4), d = (i % (HD / 4)) * 4;
+            *(float4 *) (tile + j * HD + d) = st[u];
+        }
+        __syncthreads();
+        if (j0 + 64 <= last) fetch(j0 + 64, 2);
+        if (lane >= HD || j0 > tw + R - 1) continue;
+        // 8 keys at a time; a row's keys end at its own position
+#pragma unroll 1
+        for (int c = 0; c < 64; c += 8) {
+            if (j0 + c > tw + R - 1) break;
+            double vd[8];
+            float pv[R][8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) vd[e] = (double) tile[(c + e) * HD + lane];
+#pragma unroll
+            for (int r = 0; r < R; ++r)
+#pragma unroll
+                for (int e = 0; e < 8; ++e) pv[r][e] = p[r * ts + j0 + c + e];
+            if (j0 + c + 7 <= tw) {                   // inside every row
+#pragma unroll
+                for (int e = 0; e < 8; ++e)
+#pragma unroll
+                    for (int r = 0; r < R; ++r) o[r] = fma((double) pv[r][e], vd[e], o[r]);
+            } else {
+#pragma unroll
+                for (int e = 0; e < 8; ++e)
+#pragma unroll
+                    for (int r = 0; r < R; ++r)
+                        if (j0 + c + e <= tw + r) o[r] = fma((double) pv[r][e], vd[e], o[r]);
+            }
+        }
+    }
+    if (lane < HD) {
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+            if (tw + r < T) out[(size_t) (tw + r) * os + h * HD + lane] = f2h((float) o[r]);
     }
 }
 

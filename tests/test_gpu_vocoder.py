@@ -111,6 +111,21 @@ def test_pre_transformer_attention_forms(tiny_voc, n):
     assert mx <= STAGE_TOL_MAX and rms <= STAGE_TOL_RMS, (mx, rms)
 
 
+def test_pre_transformer_attention_forms_agree(tiny_voc):
+    """Attention is causal and row-local, so the first rows of a longer call
+    equal a shorter call's bit for bit: 9,000 rows run one wave per row, 5,000
+    the 64-key tiles with one query row per wave, 65 to 400 two, up to 64 one
+    again (tile edges 1, 63, 64, 65, 127, 129)."""
+    c, w, g, o = tiny_voc
+    width = o.stages(codes_for(2, 1), 0)["input_proj"].shape[1]
+    x = (np.random.default_rng(77).standard_normal((9000, width)) * 0.5).astype(np.float32)
+    say("[gpu] pre_tfm.0 over 9000 rows")
+    want = g.run_stage("pre_tfm.0", x, 5)
+    for n in (1, 3, 63, 64, 65, 127, 129, 400, 5000):
+        say(f"[gpu] pre_tfm.0 over {n} rows")
+        assert np.array_equal(g.run_stage("pre_tfm.0", x[:n], 5), want[:n]), n
+
+
 def test_decode_window_matches_oracle(tiny_voc):
     c, w, g, o = tiny_voc
     codes = codes_for(12, 3)
