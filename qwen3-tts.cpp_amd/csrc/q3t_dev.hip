@@ -8,6 +8,7 @@
 #include "q3t_kernels.h"
 #include "q3t_frame_kernel.h"
 #include "q3t_prefill.h"
+#include "q3t_att_int.h"
 #include "q3t_streams.h"
 
 #include <hip/hip_runtime.h>
@@ -86,6 +87,10 @@ struct q3t_dev {
     float * pf_xa = nullptr, * pf_xb = nullptr, * pf_qkv = nullptr, * pf_att = nullptr;
     // f64 MFMA prefill attention: scores and probabilities [n_head][n][ls]
     float * pf_s = nullptr; uint16_t * pf_p = nullptr; size_t pf_sp_cap = 0;
+    // the digit planes of q, K and V of one layer's attention, and the number
+    // of the last attention call whose values did not fit them
+    int8_t * pf_dig = nullptr; size_t pf_dig_cap = 0;
+    int32_t * pf_wide = nullptr; int32_t pf_call = 0;
     float * pf_g = nullptr, * pf_u = nullptr, * pf_f = nullptr;
     uint16_t * pf_h = nullptr, * pf_l = nullptr;  // fp16 GEMM inputs of the fast F16 prefill (rows x kmax / ffn)
     float * pf_sc = nullptr;                      // per-row power-of-two scales of the widened ffn_down input
@@ -1943,6 +1948,27 @@ bool pf_f16_fast(const q3t_config & g) {
            g.ffn_size <= 16 * kBlock;
 }
 
+// Room for `bytes` of digit planes and the flag of values that have none; false
+// when the device has no memory for them.
+bool ensure_digits(q3t_dev * c, size_t bytes) {
+    if (!c->pf_wide) {
+        if (dev_alloc_t(c, &c->pf_wide, 1)) { (void) hipGetLastError(); return false; }
+        if (hipMemset(c->pf_wide, 0, sizeof(int32_t)) != hipSuccess) { dev_free(c, c->pf_wide); c->pf_wide = nullptr; return false; }
+    }
+    if (bytes <= c->pf_dig_cap) return true;
+    dev_free(c, c->pf_dig);
+    c->pf_dig = nullptr; c->pf_dig_cap = 0;
+    if (dev_alloc_t(c, &c->pf_dig, bytes)) { (void) hipGetLastError(); return false; }
+    c->pf_dig_cap = bytes;
+    return true;
+}
+
+// Q3T_PF_ATT_INT=0 (read per call) keeps the exact attention on the f64 MFMA.
+bool pf_att_f64() {
+    const char * e = std::getenv("Q3T_PF_ATT_INT");
+    return e && e[0] == '0';
+}
+
 // Causal attention of the n prefill rows (QKV rows in c->pf_qkv, K/V already
 // in the layer's cache) into c->pf_att.  From 64 rows on: the MFMA kernels
 // (scores, softmax, P.V; Q3T_PF_ATT_MFMA=0 keeps the row kernel), exact on f64
@@ -1981,6 +2007,26 @@ int pf_attention(q3t_dev * c, const LayerDev & L, const uint16_t * kc, const uin
     const dim3 tiles(g.n_head, (nt % 2 && nt >= 3 && !no_spread) ? nt / 2 : (nt + 1) / 2, 2);
     // q rows into the probabilities buffer's head (they are consumed before it is written)
     uint16_t * qh = c->pf_p;
+    // exact rows of an fp16 cache: int8 digits up to the row length whose
+    // scores the digit softmax holds in registers (bfloat16 values span more
+    // than four digits); without room for the digits, the f64 forms
+    const size_t qb = (size_t) g.n_head * n * 4 * kHD, kb = (size_t) g.n_kv_head * ls * 4 * kHD;
+    if (!fast && !bf && n_past + n <= pf::kIntMaxPos && !pf_att_f64() && ensure_digits(c, qb + 2 * kb)) {
+        pf::AttInt a{};
+        a.qkv = c->pf_qkv; a.qkv_stride = qkvd; a.q_norm = L.q_norm; a.eps = g.rms_eps;
+        a.rc = c->rope_cos; a.rs = c->rope_sin; a.kc = kc; a.vc = vc;
+        a.n_ctx = c->n_ctx; a.n_head = g.n_head; a.n_kv_head = g.n_kv_head; a.n = n; a.n_past = n_past; a.ls = ls;
+        a.Qh = qh; a.Qd = c->pf_dig; a.Kd = c->pf_dig + qb; a.Vd = c->pf_dig + qb + kb;
+        a.wide = c->pf_wide; a.call = c->pf_call = c->pf_call == INT32_MAX ? 1 : c->pf_call + 1;
+        hipLaunchKernelGGL(pf::k_att_split, dim3((unsigned) (n * ((g.n_head + 3) / 4) + g.n_kv_head * (ls / 64))),
+                           dim3(kBlock), 0, c->stream, a);
+        hipLaunchKernelGGL(pf::k_att_scores_int, tiles, dim3(pf::kAttT), 0, c->stream, a, scale, c->pf_s);
+        hipLaunchKernelGGL(pf::k_att_softmax_int, dim3((n + 3) / 4, g.n_head), dim3(kBlock), 0, c->stream, a, c->pf_s,
+                           c->pf_p);
+        hipLaunchKernelGGL(pf::k_att_pv_int, tiles, dim3(pf::kAttT), 0, c->stream, a, (const int8_t *) c->pf_s,
+                           (const uint16_t *) c->pf_p, c->pf_att, qd);
+        return 0;
+    }
     hipLaunchKernelGGL(pf::k_att_q, dim3(n, (g.n_head + 3) / 4), dim3(kBlock), 0, c->stream, (const float *) c->pf_qkv,
                        qkvd, L.q_norm, g.rms_eps, (const float *) c->rope_cos, (const float *) c->rope_sin, n, n_past,
                        g.n_head, qh, bf);

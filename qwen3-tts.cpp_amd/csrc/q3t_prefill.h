@@ -886,11 +886,10 @@ __global__ __launch_bounds__(kAttT) void k_att_scores_fast(const uint16_t * __re
                                                             int32_t n_past, float scale, float * __restrict__ S,
                                                             int32_t ls, int32_t bf);
 
-__global__ __launch_bounds__(kAttT) void k_att_scores(const uint16_t * __restrict__ Qh,
-                                                       const uint16_t * __restrict__ kc, int32_t n_ctx, int32_t n_head,
-                                                       int32_t n_kv_head, int32_t n, int32_t n_past, float scale,
-                                                       float * __restrict__ S, int32_t ls, int32_t bf) {
-    __shared__ __align__(16) uint16_t kt[2][kAT * kKS];
+__device__ __forceinline__ void att_scores_body(const uint16_t * __restrict__ Qh, const uint16_t * __restrict__ kc,
+                                                int32_t n_ctx, int32_t n_head, int32_t n_kv_head, int32_t n,
+                                                int32_t n_past, float scale, float * __restrict__ S, int32_t ls,
+                                                int32_t bf, uint16_t (*kt)[kAT * kKS]) {
     const int h = blockIdx.x, tiles = (n + kAT - 1) / kAT, g = h / (n_head / n_kv_head), grp = blockIdx.z;
     const int t = threadIdx.x, w = t >> 6, l = t & 63, i = l & 15, k = l >> 4;
     const int krow = t >> 4, kch = t & 15;                  // staging: positions krow + 16u, 8-dim chunk
@@ -972,6 +971,14 @@ __global__ __launch_bounds__(kAttT) void k_att_scores(const uint16_t * __restric
             __syncthreads();
         }
     }
+}
+
+__global__ __launch_bounds__(kAttT) void k_att_scores(const uint16_t * __restrict__ Qh,
+                                                       const uint16_t * __restrict__ kc, int32_t n_ctx, int32_t n_head,
+                                                       int32_t n_kv_head, int32_t n, int32_t n_past, float scale,
+                                                       float * __restrict__ S, int32_t ls, int32_t bf) {
+    __shared__ __align__(16) uint16_t kt[2][kAT * kKS];
+    att_scores_body(Qh, kc, n_ctx, n_head, n_kv_head, n, n_past, scale, S, ls, bf, kt);
 }
 
 // The fast form of k_att_scores (see its declaration); same grid, tile
@@ -1095,13 +1102,8 @@ __device__ __forceinline__ void softmax_row_reg(const float * __restrict__ sr, u
 // position row is not the three-read straggler that ends the launch, and the
 // kernel keeps 64 VGPRs, eight waves per SIMD); longer rows are read three
 // times.
-__global__ __launch_bounds__(kBlock) void k_att_softmax(const float * __restrict__ S, int32_t n, int32_t n_past,
-                                                        int32_t ls, uint16_t * __restrict__ P, int32_t bf) {
-    const int lane = threadIdx.x & 63, row = blockIdx.x * 4 + (threadIdx.x >> 6), h = blockIdx.y;
-    if (row >= n) return;                   // whole wave
-    const int cnt = n_past + row + 1;
-    const float * sr = S + ((size_t) h * n + row) * ls;
-    uint16_t * pr = P + ((size_t) h * n + row) * ls;
+__device__ __forceinline__ void att_softmax_row(const float * __restrict__ sr, uint16_t * __restrict__ pr, int cnt,
+                                                int lane, int bf) {
     if (cnt <= 64 * 16) { softmax_row_reg<16>(sr, pr, cnt, lane, bf); return; }
     if (cnt <= 64 * 32) { softmax_row_reg<32>(sr, pr, cnt, lane, bf); return; }
     if (cnt <= 64 * 40) { softmax_row_reg<40>(sr, pr, cnt, lane, bf); return; }
@@ -1112,6 +1114,14 @@ __global__ __launch_bounds__(kBlock) void k_att_softmax(const float * __restrict
     for (int j = lane; j < cnt; j += 64) sum += (double) expf_q3t(sr[j] - mx);
     const float inv = (float) (1.0 / wave_sum_d(sum));
     for (int j = lane; j < cnt; j += 64) pr[j] = f2kv(expf_q3t(sr[j] - mx) * inv, bf);
+}
+
+__global__ __launch_bounds__(kBlock) void k_att_softmax(const float * __restrict__ S, int32_t n, int32_t n_past,
+                                                        int32_t ls, uint16_t * __restrict__ P, int32_t bf) {
+    const int lane = threadIdx.x & 63, row = blockIdx.x * 4 + (threadIdx.x >> 6), h = blockIdx.y;
+    if (row >= n) return;                   // whole wave
+    const size_t at = ((size_t) h * n + row) * ls;
+    att_softmax_row(S + at, P + at, n_past + row + 1, lane, bf);
 }
 
 // grid (n_head, Y, 2), tiles paired as in k_att_scores; grid z = grp takes
@@ -1129,12 +1139,11 @@ __global__ __launch_bounds__(kBlock) void k_att_softmax(const float * __restrict
 // Probabilities past a row's last position, and V rows past the tile's last
 // position, are staged as zero.
 constexpr int kVN = 64 + 8;      // LDS row stride (halves) of a staged V half-tile: conflict-free 16-byte writes
-__global__ __launch_bounds__(kAttT, 4) void k_att_pv(const uint16_t * __restrict__ P, int32_t ls,
-                                                   const uint16_t * __restrict__ vc, int32_t n_ctx, int32_t n_head,
-                                                   int32_t n_kv_head, int32_t n, int32_t n_past,
-                                                   float * __restrict__ out, int32_t out_stride, int32_t bf) {
-    __shared__ __align__(16) uint16_t pt[2][kAT * kVS];      // [row][position]
-    __shared__ __align__(16) uint16_t vt[2][kAT * kVN];      // [position][dim - 64 grp]
+__device__ __forceinline__ void att_pv_body(const uint16_t * __restrict__ P, int32_t ls,
+                                            const uint16_t * __restrict__ vc, int32_t n_ctx, int32_t n_head,
+                                            int32_t n_kv_head, int32_t n, int32_t n_past, float * __restrict__ out,
+                                            int32_t out_stride, int32_t bf, uint16_t (*pt)[kAT * kVS],
+                                            uint16_t (*vt)[kAT * kVN]) {
     const int h = blockIdx.x, tiles = (n + kAT - 1) / kAT, g = h / (n_head / n_kv_head), grp = blockIdx.z;
     const int t = threadIdx.x, w = t >> 6, l = t & 63, i = l & 15, k = l >> 4;
     const int srow = t >> 3, sch = t & 7;                    // staging: rows / positions srow + 32u, 8-wide chunk
@@ -1235,6 +1244,15 @@ __global__ __launch_bounds__(kAttT, 4) void k_att_pv(const uint16_t * __restrict
         }
     }
   }
+}
+
+__global__ __launch_bounds__(kAttT, 4) void k_att_pv(const uint16_t * __restrict__ P, int32_t ls,
+                                                   const uint16_t * __restrict__ vc, int32_t n_ctx, int32_t n_head,
+                                                   int32_t n_kv_head, int32_t n, int32_t n_past,
+                                                   float * __restrict__ out, int32_t out_stride, int32_t bf) {
+    __shared__ __align__(16) uint16_t pt[2][kAT * kVS];      // [row][position]
+    __shared__ __align__(16) uint16_t vt[2][kAT * kVN];      // [position][dim - 64 grp]
+    att_pv_body(P, ls, vc, n_ctx, n_head, n_kv_head, n, n_past, out, out_stride, bf, pt, vt);
 }
 
 // The fast form of k_att_pv: P.V on 16x16x32 fp16 (bfloat16) MFMAs with
