@@ -1800,33 +1800,31 @@ int ensure_pf(q3t_dev * c, int n) {
     return 0;
 }
 
+// With w2 / y2 a second matrix of the same shape in the same launch.
 void pf_gemm(q3t_dev * c, const Slot & w, int N, int K, int n, float * y, const float * res, int rs = -1,
-             const int8_t * q = nullptr, const float * dx = nullptr) {
-    // tile: 64 weight rows x 32 JT tokens, JT = 2 unless that leaves the launch
-    // with fewer workgroups than CUs; two Q8_0 blocks per stage
-    int IR = 2, JT = 2, GB = 2;
-    while (JT > 1 && (int64_t) (N / (32 * IR)) * ((n + 32 * JT - 1) / (32 * JT)) < c->n_cu) JT >>= 1;
-    if (const char * e = std::getenv("Q3T_PF_TILE")) {      // "<IR>x<JT>x<GB>"
-        const int ir = e[0] - '0', jt = e[1] == 'x' ? e[2] - '0' : 0, gb = e[1] == 'x' && e[3] == 'x' ? e[4] - '0' : 2;
-        if ((ir == 2 || (ir == 4 && N % 128 == 0 && gb == 2)) && (jt == 1 || jt == 2 || jt == 4) &&
-            (gb == 2 || gb == 4) && (K / kQK) % gb == 0) { IR = ir; JT = jt; GB = gb; }
-    }
-    const dim3 grid(N / (32 * IR), (n + 32 * JT - 1) / (32 * JT));
+             const int8_t * q = nullptr, const float * dx = nullptr, const Slot * w2 = nullptr, float * y2 = nullptr) {
     const int8_t * qq = q ? q : (const int8_t *) c->pf_q;
     const float * dd = dx ? dx : (const float *) c->pf_dx;
     const int epi = res ? (int) EPI_RESID : (int) EPI_STORE;
-    const int r = rs < 0 ? N : rs;
-#define Q3T_PF_GEMM(ir, jt, gb)                                                                                  \
-    hipLaunchKernelGGL((pf::k_gemm_q8<ir, jt, gb>), grid, dim3(kBlock), 0, c->stream, (const int8_t *) w.data, \
-                       (const uint16_t *) w.scales, N, K, qq, dd, n, y, N, res, r, epi)
-#define Q3T_PF_GEMM_JT(ir, gb)                                                                                   \
-    if (JT == 4) Q3T_PF_GEMM(ir, 4, gb); else if (JT == 2) Q3T_PF_GEMM(ir, 2, gb); else Q3T_PF_GEMM(ir, 1, gb)
-    if (GB == 4) {
-        Q3T_PF_GEMM_JT(2, 4);
-    } else {
-        if (IR == 4) { Q3T_PF_GEMM_JT(4, 2); } else { Q3T_PF_GEMM_JT(2, 2); }
-    }
-#undef Q3T_PF_GEMM_JT
+    const int r = rs < 0 ? N : rs, m = w2 ? 2 : 1;
+    const int8_t * wb = w2 ? (const int8_t *) w2->data : nullptr;
+    const uint16_t * wbd = w2 ? (const uint16_t *) w2->scales : nullptr;
+#define Q3T_PF_GEMM(rt, jt, wr, wt, gb)                                                                           \
+    hipLaunchKernelGGL((pf::k_gemm_q8<rt, jt, wr, wt, gb>),                                                       \
+                       dim3(m * N / (16 * rt * wr), (n + 16 * jt * wt - 1) / (16 * jt * wt)), dim3(kBlock), 0,    \
+                       c->stream, (const int8_t *) w.data, (const uint16_t *) w.scales, N, K, qq, dd, n, y, N,    \
+                       res, r, epi, wb, wbd, y2)
+    // 64 x 64 tiles from 3.5 workgroups per CU on (all four resident at once);
+    // 64 x 32 with the blocks of a stage over two wave pairs down to 1.5 per
+    // CU; then 32 x 32.  Measured either side of the lines (us): 800 rows of
+    // 4096 x 1024 (3.3 per CU) 25.7 / 25.1, 1,200 rows of 3072 x 1024 (3.6)
+    // 25.8 / 27.1; 209 rows of 4096 x 1024 (1.75) 10.4 / 10.7, of 3072 x 1024
+    // (1.3) 10.1 / 9.0.
+    const int64_t t64 = (int64_t) (m * N / 64) * ((n + 63) / 64), t32 = (int64_t) (m * N / 64) * ((n + 31) / 32);
+    if (2 * t64 >= 7 * c->n_cu) Q3T_PF_GEMM(2, 2, 2, 2, 4);
+    else if (2 * t32 >= 3 * c->n_cu) Q3T_PF_GEMM(2, 2, 2, 1, 4);
+    else if (K % 256 == 0) Q3T_PF_GEMM(1, 2, 2, 1, 8);
+    else Q3T_PF_GEMM(1, 2, 2, 1, 4);
 #undef Q3T_PF_GEMM
 }
 
@@ -2129,8 +2127,7 @@ int prefill_mfma(q3t_dev * c, int n, int n_past) {
         pf_quant(c, c->pf_att, n, qd, nullptr);
         pf_gemm(c, L.wo, d, qd, n, c->pf_xb, x);
         pf_quant(c, c->pf_xb, n, d, L.ffn_norm);
-        pf_gemm(c, L.wg, ffn, d, n, c->pf_g, nullptr);
-        pf_gemm(c, L.wu, ffn, d, n, c->pf_u, nullptr);
+        pf_gemm(c, L.wg, ffn, d, n, c->pf_g, nullptr, -1, nullptr, nullptr, &L.wu, c->pf_u);
         pf_quant(c, c->pf_g, n, ffn, nullptr, -1, nullptr, nullptr, c->pf_u);   // SwiGLU fused into the quantisation
         pf_gemm(c, L.wd, d, ffn, n, c->pf_xa, c->pf_xb);
         x = c->pf_xa;

@@ -82,166 +82,205 @@ __global__ __launch_bounds__(kBlock) void k_quant_rows(const float * __restrict_
 }
 
 // Y[t][r] = epi(sum_b fp16(dw[r][b]) * dx[t][b] * sum_k W[r][32b+k] Q[t][32b+k])
-// on a (32 IR rows) x (32 JT tokens) tile per workgroup: wave (wr, wt) =
-// (wave & 1, wave >> 1) owns IR x JT MFMA tiles of 16 x 16.  Each stage holds
-// kGB Q8_0 blocks of the tile's weight and activation rows in LDS (rows padded
-// by 8 bytes against bank conflicts) with their scales, double-buffered: the
-// next stage's global loads are in flight during this stage's MFMAs.  MFMA
-// lane layout (16x16x32 i8): A[m = l%16][k = 8(l/16)..+7], B[k][n = l%16],
-// D[m = 4(l/16)+i][n = l%16]; each block's exact int32 sums take the fp16 x
-// fp16 scale product (exact in fp32) in an fp64 fma, so the fp64 sum of exact
-// terms is rounded to fp32 once.  epi: EPI_STORE or EPI_RESID (res [n][rs],
-// rs = 0 broadcasts one row).  Requires N % (32 IR) == 0, K % (32 kGB) == 0.
-// A wave skips the MFMAs and epilogue of its 16-token groups that lie wholly
-// past n, so the partial last token tile (2,049 rows: one row) costs about
-// half a tile, not a whole one.
-template <int IR, int JT, int GB>
+// on a tile of TN weight rows x TM tokens per workgroup; grid x beyond N / TN
+// takes a second matrix of the same shape (gate and up in one launch).  WR x
+// WT waves share the tile, each RT x JT MFMA tiles of 16 x 16; the 4 / (WR WT)
+// waves left split the Q8_0 blocks of a stage and add their fp64 sums through
+// LDS in wave order.  Each stage holds GB blocks of the tile's weight and
+// activation rows in LDS (rows padded by 8 bytes against bank conflicts) with
+// their scales, double-buffered: the next stage's global loads are in flight
+// during this stage's MFMAs.  MFMA lane layout (16x16x32 i8): A[m = l%16][k =
+// 8(l/16)..+7], B[k][n = l%16], D[m = 4(l/16)+i][n = l%16]; each block's exact
+// int32 sums take the fp16 x fp16 scale product (exact in fp32) in an fp64
+// fma, so the fp64 sum of exact terms is rounded to fp32 once.  epi: EPI_STORE
+// or EPI_RESID (res [n][rs], rs = 0 broadcasts one row).  Tokens past n repeat
+// row n - 1 and store nothing; a wave whose tokens all lie past n skips the
+// arithmetic.  Requires N % TN == 0, K % (32 GB) == 0.
+//
+// Bound by the vector ALU at large n: a block's 64 outputs take a multiply,
+// two conversions and an fma, 17 clocks of the 22-25 measured.  One branch
+// per MFMA tile (skipping 16-token groups past n) had kept the compiler from
+// overlapping an MFMA with the epilogue before it.  Few rows are a chain of
+// stages, so their blocks go to several waves.  One GEMM, us, before -> now:
+// 1,600 rows QKV 47 -> 41, Wo 43 -> 29, down 62 -> 40; 209 rows QKV 17.5 ->
+// 10.4, Wo 27 -> 8.3, down 39 -> 11.
+template <int RT, int JT, int WR, int WT, int GB>
 struct Q8Tile {
-    static constexpr int TN = 32 * IR, TM = 32 * JT;
-    static constexpr int ROWB = GB * kQK + 8;          // bytes per staged row (padded against bank conflicts)
+    static constexpr int KW = 4 / (WR * WT);           // waves along K
+    static constexpr int TN = 16 * RT * WR, TM = 16 * JT * WT;
+    static constexpr int ROWB = GB * kQK + 8;
     static constexpr int A_BYTES = TN * ROWB, B_BYTES = TM * ROWB;
-    static constexpr int STAGE = A_BYTES + B_BYTES + (TN + TM) * GB * 4;
-    static constexpr int LDS = 2 * STAGE;
+    static constexpr int DW_BYTES = GB * TN * 4, DX_BYTES = GB * TM * 4;
+    static constexpr int STAGE = A_BYTES + B_BYTES + DW_BYTES + DX_BYTES;
+    static constexpr int RED = KW > 1 ? (KW - 1) * RT * JT * 64 * 32 * WR * WT : 0;
+    static constexpr int LDS = 2 * STAGE > RED ? 2 * STAGE : RED;
 };
 
-template <int IR, int JT, int kGB>
+template <int RT, int JT, int WR, int WT, int GB>
 __global__ __launch_bounds__(kBlock) void k_gemm_q8(const int8_t * __restrict__ W, const uint16_t * __restrict__ Wd,
                                                     int32_t N, int32_t K, const int8_t * __restrict__ Q,
                                                     const float * __restrict__ dx, int32_t n, float * __restrict__ Y,
-                                                    int32_t ys, const float * __restrict__ res, int32_t rs, int32_t epi) {
-    using T = Q8Tile<IR, JT, kGB>;
-    constexpr int kRowB = T::ROWB;
+                                                    int32_t ys, const float * __restrict__ res, int32_t rs, int32_t epi,
+                                                    const int8_t * __restrict__ W2, const uint16_t * __restrict__ Wd2,
+                                                    float * __restrict__ Y2) {
+    using T = Q8Tile<RT, JT, WR, WT, GB>;
+    constexpr int KW = T::KW, kRowB = T::ROWB, TN = T::TN, TM = T::TM;
     __shared__ __align__(16) char smem[T::LDS];
-    const int BPR = K / kQK, S = BPR / kGB;
-    const int r0 = blockIdx.x * T::TN, t0 = blockIdx.y * T::TM;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, wr = wave & 1, wt = wave >> 1;
+    const int BPR = K / kQK, S = BPR / GB;
+    const int nx = N / TN, t0 = blockIdx.y * TM;
+    int bx = blockIdx.x;
+    if (bx >= nx) { bx -= nx; W = W2; Wd = Wd2; Y = Y2; }
+    const int r0 = bx * TN;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wr = wave % WR, wt = (wave / WR) % WT, wk = wave / (WR * WT);
     const int lm = lane & 15, lk = lane >> 4;
-    // staging: 16-byte chunks, kGB * 2 per row (A then B rows), scale pairs
-    constexpr int CPR = kGB * kQK / 16;                  // chunks per row
-    constexpr int NA = (T::TN * CPR + kBlock - 1) / kBlock, NB = (T::TM * CPR + kBlock - 1) / kBlock;
-    int4 ra[NA], rb[NB];
-    float sw[kGB], sx[kGB];
-#pragma unroll
-    for (int g = 0; g < kGB; ++g) { sw[g] = 0.f; sx[g] = 0.f; }
+    constexpr int CPR = GB * 2;                          // 16-byte chunks per row
+    constexpr int NA = TN * CPR / kBlock > 0 ? TN * CPR / kBlock : 1, NB = TM * CPR / kBlock > 0 ? TM * CPR / kBlock : 1;
+    static_assert((TN * CPR) % kBlock == 0 || TN * CPR < kBlock, "whole rounds");
+    static_assert((TM * CPR) % kBlock == 0 || TM * CPR < kBlock, "whole rounds");
+    v4i ra[NA], rb[NB];
+    typedef uint16_t hv __attribute__((ext_vector_type(GB)));
+    typedef float fv __attribute__((ext_vector_type(GB)));
+    hv sw;
+    fv sx;
     auto fetch = [&](int st) {
-        const int kb = st * kGB;
+        const int kb = st * GB;
 #pragma unroll
         for (int i = 0; i < NA; ++i) {
-            const int c = tid + i * kBlock, row = c / CPR, col = c - row * CPR;
-            ra[i] = c < T::TN * CPR ? *(const int4 *) (W + (size_t) (r0 + row) * K + kb * kQK + col * 16) : make_int4(0, 0, 0, 0);
+            const int c = tid + i * kBlock, row = (c / CPR) % TN, col = c % CPR;
+            ra[i] = *(const v4i *) (W + (size_t) (r0 + row) * K + kb * kQK + col * 16);
         }
 #pragma unroll
         for (int i = 0; i < NB; ++i) {
-            const int c = tid + i * kBlock, row = c / CPR, col = c - row * CPR;
-            const int tok = t0 + row;
-            rb[i] = (c < T::TM * CPR && tok < n) ? *(const int4 *) (Q + (size_t) tok * K + kb * kQK + col * 16)
-                                                 : make_int4(0, 0, 0, 0);
+            const int c = tid + i * kBlock, row = (c / CPR) % TM, col = c % CPR;
+            rb[i] = *(const v4i *) (Q + (size_t) min(t0 + row, n - 1) * K + kb * kQK + col * 16);
         }
-        if (tid < T::TN) {
-            const uint16_t * p = Wd + (size_t) (r0 + tid) * BPR + kb;
-#pragma unroll
-            for (int g = 0; g < kGB; ++g) sw[g] = h2f(p[g]);
-        }
-        if (tid < T::TM) {
-            const int tok = t0 + tid;
-#pragma unroll
-            for (int g = 0; g < kGB; ++g) sx[g] = tok < n ? dx[(size_t) tok * BPR + kb + g] : 0.f;
-        }
+        sw = *(const hv *) (Wd + (size_t) (r0 + tid % TN) * BPR + kb);
+        sx = *(const fv *) (dx + (size_t) min(t0 + tid % TM, n - 1) * BPR + kb);
     };
     auto stash = [&](int buf) {
         char * st = smem + buf * T::STAGE;
 #pragma unroll
         for (int i = 0; i < NA; ++i) {
-            const int c = tid + i * kBlock, row = c / CPR, col = c - row * CPR;
-            if (c < T::TN * CPR) {
-                long * d = (long *) (st + row * kRowB + col * 16);   // 8-byte aligned rows
+            const int c = tid + i * kBlock, row = c / CPR, col = c % CPR;
+            if (TN * CPR >= kBlock || c < TN * CPR) {
+                long * d = (long *) (st + row * kRowB + col * 16);
                 d[0] = ((const long *) &ra[i])[0];
                 d[1] = ((const long *) &ra[i])[1];
             }
         }
 #pragma unroll
         for (int i = 0; i < NB; ++i) {
-            const int c = tid + i * kBlock, row = c / CPR, col = c - row * CPR;
-            if (c < T::TM * CPR) {
+            const int c = tid + i * kBlock, row = c / CPR, col = c % CPR;
+            if (TM * CPR >= kBlock || c < TM * CPR) {
                 long * d = (long *) (st + T::A_BYTES + row * kRowB + col * 16);
                 d[0] = ((const long *) &rb[i])[0];
                 d[1] = ((const long *) &rb[i])[1];
             }
         }
-        float * sdw = (float *) (st + T::A_BYTES + T::B_BYTES);   // [kGB][TN]
-        float * sdx = sdw + kGB * T::TN;                          // [kGB][TM]
+        float * sdw = (float *) (st + T::A_BYTES + T::B_BYTES);     // [GB][TN]
+        float * sdx = sdw + GB * TN;                      // [GB][TM]
+        if (tid < TN) {
 #pragma unroll
-        for (int g = 0; g < kGB; ++g) {
-            if (tid < T::TN) sdw[g * T::TN + tid] = sw[g];
-            if (tid < T::TM) sdx[g * T::TM + tid] = sx[g];
+            for (int g = 0; g < GB; ++g) sdw[g * TN + tid] = h2f(sw[g]);
+        }
+        if (tid < TM) {
+#pragma unroll
+            for (int g = 0; g < GB; ++g) sdx[g * TM + tid] = sx[g];
         }
     };
-
-    double acc[IR][JT][4];
+    double acc[RT][JT][4];
 #pragma unroll
-    for (int i = 0; i < IR; ++i)
+    for (int i = 0; i < RT; ++i)
 #pragma unroll
         for (int j = 0; j < JT; ++j)
 #pragma unroll
             for (int e = 0; e < 4; ++e) acc[i][j][e] = 0.0;
-    const v4i zero = {0, 0, 0, 0};
-
-    fetch(0);
-    stash(0);
-    __syncthreads();
-    for (int st = 0; st < S; ++st) {
-        const int buf = st & 1;
-        if (st + 1 < S) fetch(st + 1);
+    const bool live = t0 + wt * JT * 16 < n;
+    auto compute = [&](int buf) {
+        if (!live) return;
         const char * sb = smem + buf * T::STAGE;
         const float * sdw = (const float *) (sb + T::A_BYTES + T::B_BYTES);
-        const float * sdx = sdw + kGB * T::TN;
+        const float * sdx = sdw + GB * TN;
 #pragma unroll
-        for (int kb = 0; kb < kGB; ++kb) {
+        for (int kq = 0; kq < GB / KW; ++kq) {
+            const int kb = kq * KW + wk;
             long bq[JT];
             float dxv[JT];
 #pragma unroll
             for (int j = 0; j < JT; ++j) {
-                const int tl = wt * JT * 16 + j * 16 + lm;
+                const int tl = (wt * JT + j) * 16 + lm;
                 bq[j] = *(const long *) (sb + T::A_BYTES + tl * kRowB + kb * kQK + 8 * lk);
-                dxv[j] = sdx[kb * T::TM + tl];
+                dxv[j] = sdx[kb * TM + tl];
             }
 #pragma unroll
-            for (int i = 0; i < IR; ++i) {
-                const int rl = wr * IR * 16 + i * 16;
+            for (int i = 0; i < RT; ++i) {
+                const int rl = (wr * RT + i) * 16;
                 const long a = *(const long *) (sb + (rl + lm) * kRowB + kb * kQK + 8 * lk);
-                float dwv[4];
+                const float4 dw = *(const float4 *) (sdw + kb * TN + rl + 4 * lk);
+                const float dwv[4] = {dw.x, dw.y, dw.z, dw.w};
+                v4i d[JT];
 #pragma unroll
-                for (int e = 0; e < 4; ++e) dwv[e] = sdw[kb * T::TN + rl + 4 * lk + e];
+                for (int j = 0; j < JT; ++j) d[j] = __builtin_amdgcn_mfma_i32_16x16x32_i8(a, bq[j], v4i{0, 0, 0, 0}, 0, 0, 0);
 #pragma unroll
-                for (int j = 0; j < JT; ++j) {
-                    if (t0 + (wt * JT + j) * 16 >= n) continue;   // 16 tokens past n (wave-uniform): nothing to add
-                    const v4i d = __builtin_amdgcn_mfma_i32_16x16x32_i8(a, bq[j], zero, 0, 0, 0);
-                    // fp16 x fp16 scale product exact in fp32; times the int32 block sum exact in fp64
+                for (int j = 0; j < JT; ++j)
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) acc[i][j][e] = fma((double) (dwv[e] * dxv[j]), (double) d[e], acc[i][j][e]);
-                }
+                    for (int e = 0; e < 4; ++e) acc[i][j][e] = fma((double) (dwv[e] * dxv[j]), (double) d[j][e], acc[i][j][e]);
             }
         }
-        if (st + 1 < S) stash(buf ^ 1);
+    };
+    fetch(0);
+    stash(0);
+    __syncthreads();
+    for (int st = 0; st < S; ++st) {
+        if (st + 1 < S) fetch(st + 1);
+        compute(st & 1);
+        // the next stage's LDS stores (and so the wait for its loads) stay behind this stage's arithmetic
+        __asm__ volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+        if (st + 1 < S) stash((st + 1) & 1);
         __syncthreads();
+    }
+    if constexpr (KW > 1) {
+        double * red = (double *) smem;
+        const int wq = wave % (WR * WT);
+        if (wk > 0) {
+#pragma unroll
+            for (int i = 0; i < RT; ++i)
+#pragma unroll
+                for (int j = 0; j < JT; ++j)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        red[(((((wk - 1) * WR * WT + wq) * RT + i) * JT + j) * 4 + e) * 64 + lane] = acc[i][j][e];
+        }
+        __syncthreads();
+        if (wk > 0) return;
+#pragma unroll
+        for (int k = 1; k < KW; ++k)
+#pragma unroll
+            for (int i = 0; i < RT; ++i)
+#pragma unroll
+                for (int j = 0; j < JT; ++j)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        acc[i][j][e] += red[(((((k - 1) * WR * WT + wq) * RT + i) * JT + j) * 4 + e) * 64 + lane];
     }
 #pragma unroll
     for (int j = 0; j < JT; ++j) {
-        const int tok = t0 + wt * JT * 16 + j * 16 + lm;
+        const int tok = t0 + (wt * JT + j) * 16 + lm;
         if (tok >= n) continue;
 #pragma unroll
-        for (int i = 0; i < IR; ++i) {
-            const int r = r0 + wr * IR * 16 + i * 16 + 4 * lk;
+        for (int i = 0; i < RT; ++i) {
+            const int r = r0 + (wr * RT + i) * 16 + 4 * lk;
             float4 v = make_float4((float) acc[i][j][0], (float) acc[i][j][1], (float) acc[i][j][2], (float) acc[i][j][3]);
             if (epi == EPI_RESID) {
-                const float * rr = res + (size_t) tok * rs + r;
-                v.x = v.x + rr[0]; v.y = v.y + rr[1]; v.z = v.z + rr[2]; v.w = v.w + rr[3];
+                const float * q = res + (size_t) tok * rs + r;
+                v.x = v.x + q[0]; v.y = v.y + q[1]; v.z = v.z + q[2]; v.w = v.w + q[3];
             }
             *(float4 *) (Y + (size_t) tok * ys + r) = v;
         }
     }
 }
-
 
 constexpr int kTile = 64;         // output rows and tokens per workgroup of the F16 GEMM
 
