@@ -8,6 +8,7 @@
 #include "q3t_kernels.h"
 #include "q3t_frame_kernel.h"
 #include "q3t_prefill.h"
+#include "q3t_att_flash.h"
 #include "q3t_att_int.h"
 #include "q3t_streams.h"
 
@@ -1946,9 +1947,17 @@ bool pf_f16_fast(const q3t_config & g) {
            g.ffn_size <= 16 * kBlock;
 }
 
-// Room for `bytes` of digit planes and the flag of values that have none; false
-// when the device has no memory for them.
-bool ensure_digits(q3t_dev * c, size_t bytes) {
+// fp16(x) of n contiguous rows of K.
+void pf_rows_h16(q3t_dev * c, const float * x, int K, int n, uint16_t * y) {
+    const size_t cnt = (size_t) n * K;
+    hipLaunchKernelGGL(pf::k_rows_h16, dim3((unsigned) std::min<size_t>((cnt + kBlock - 1) / kBlock, 4096)), dim3(kBlock),
+                       0, c->stream, x, K, K, n, y);
+}
+
+// Room for `bytes` of attention operands (the digit planes, or the fast form's q
+// rows and V^T tiles) and the flag of values that have no digits; false when the
+// device has no memory for them.
+bool ensure_operands(q3t_dev * c, size_t bytes) {
     if (!c->pf_wide) {
         if (dev_alloc_t(c, &c->pf_wide, 1)) { (void) hipGetLastError(); return false; }
         if (hipMemset(c->pf_wide, 0, sizeof(int32_t)) != hipSuccess) { dev_free(c, c->pf_wide); c->pf_wide = nullptr; return false; }
@@ -1968,10 +1977,11 @@ bool pf_att_f64() {
 }
 
 // Causal attention of the n prefill rows (QKV rows in c->pf_qkv, K/V already
-// in the layer's cache) into c->pf_att.  From 64 rows on: the MFMA kernels
-// (scores, softmax, P.V; Q3T_PF_ATT_MFMA=0 keeps the row kernel), exact on f64
-// MFMA or, fast, on fp16 (bfloat16) MFMA with fp32 accumulation; below, or
-// when the scores would not fit 4 GiB, one workgroup per row.
+// in the layer's cache) into c->pf_att; fast, into the fp16 rows c->pf_h.  From
+// 64 rows on: fast, one kernel on fp16 (bfloat16) MFMA with fp32 accumulation,
+// else the exact MFMA kernels (scores, softmax, P.V; Q3T_PF_ATT_MFMA=0 keeps
+// the row kernel); below, or when the exact kernels' scores would not fit 4 GiB,
+// one workgroup per row.
 int pf_attention(q3t_dev * c, const LayerDev & L, const uint16_t * kc, const uint16_t * vc, int n, int n_past,
                  bool fast) {
     const q3t_config & g = c->cfg;
@@ -1986,6 +1996,21 @@ int pf_attention(q3t_dev * c, const LayerDev & L, const uint16_t * kc, const uin
                            c->stream, (const float *) c->pf_qkv, qkvd, L.q_norm, g.rms_eps, (const float *) c->rope_cos,
                            (const float *) c->rope_sin, kc, vc, c->n_ctx, g.n_head, g.n_kv_head, n_past, scale,
                            c->pf_att, qd, bf);
+        if (fast) pf_rows_h16(c, c->pf_att, qd, n, c->pf_h);
+        return 0;
+    }
+    if (fast) {
+        const size_t qb = (size_t) g.n_head * n * kHD, vb = (size_t) g.n_kv_head * ls * kHD;
+        if (!ensure_operands(c, 2 * (qb + vb))) return -1;
+        pf::AttFlash a{};
+        a.qkv = c->pf_qkv; a.qkv_stride = qkvd; a.q_norm = L.q_norm; a.eps = g.rms_eps;
+        a.rc = c->rope_cos; a.rs = c->rope_sin; a.kc = kc; a.vc = vc;
+        a.n_ctx = c->n_ctx; a.n_head = g.n_head; a.n_kv_head = g.n_kv_head; a.n = n; a.n_past = n_past; a.bf = bf;
+        a.Qh = (uint16_t *) c->pf_dig; a.Vt = a.Qh + qb;
+        hipLaunchKernelGGL(pf::k_att_flash_in, dim3((unsigned) (n * ((g.n_head + 3) / 4) + g.n_kv_head * (ls / 64))),
+                           dim3(kBlock), 0, c->stream, a);
+        hipLaunchKernelGGL(pf::k_att_flash, dim3(g.n_head, (n + pf::kAT - 1) / pf::kAT), dim3(pf::kFT), 0, c->stream, a,
+                           scale * 1.44269504088896341f, c->pf_h, qd);
         return 0;
     }
     // the probabilities buffer also holds the q rows [n_head][n][128] first
@@ -2009,7 +2034,7 @@ int pf_attention(q3t_dev * c, const LayerDev & L, const uint16_t * kc, const uin
     // scores the digit softmax holds in registers (bfloat16 values span more
     // than four digits); without room for the digits, the f64 forms
     const size_t qb = (size_t) g.n_head * n * 4 * kHD, kb = (size_t) g.n_kv_head * ls * 4 * kHD;
-    if (!fast && !bf && n_past + n <= pf::kIntMaxPos && !pf_att_f64() && ensure_digits(c, qb + 2 * kb)) {
+    if (!bf && n_past + n <= pf::kIntMaxPos && !pf_att_f64() && ensure_operands(c, qb + 2 * kb)) {
         pf::AttInt a{};
         a.qkv = c->pf_qkv; a.qkv_stride = qkvd; a.q_norm = L.q_norm; a.eps = g.rms_eps;
         a.rc = c->rope_cos; a.rs = c->rope_sin; a.kc = kc; a.vc = vc;
@@ -2028,11 +2053,11 @@ int pf_attention(q3t_dev * c, const LayerDev & L, const uint16_t * kc, const uin
     hipLaunchKernelGGL(pf::k_att_q, dim3(n, (g.n_head + 3) / 4), dim3(kBlock), 0, c->stream, (const float *) c->pf_qkv,
                        qkvd, L.q_norm, g.rms_eps, (const float *) c->rope_cos, (const float *) c->rope_sin, n, n_past,
                        g.n_head, qh, bf);
-    hipLaunchKernelGGL(fast ? pf::k_att_scores_fast : pf::k_att_scores, tiles, dim3(pf::kAttT), 0, c->stream,
+    hipLaunchKernelGGL(pf::k_att_scores, tiles, dim3(pf::kAttT), 0, c->stream,
                        (const uint16_t *) qh, kc, c->n_ctx, g.n_head, g.n_kv_head, n, n_past, scale, c->pf_s, ls, bf);
     hipLaunchKernelGGL(pf::k_att_softmax, dim3((n + 3) / 4, g.n_head), dim3(kBlock), 0, c->stream,
                        (const float *) c->pf_s, n, n_past, ls, c->pf_p, bf);
-    hipLaunchKernelGGL(fast ? pf::k_att_pv_fast : pf::k_att_pv, tiles, dim3(pf::kAttT), 0, c->stream,
+    hipLaunchKernelGGL(pf::k_att_pv, tiles, dim3(pf::kAttT), 0, c->stream,
                        (const uint16_t *) c->pf_p, ls, vc, c->n_ctx, g.n_head, g.n_kv_head, n, n_past, c->pf_att, qd, bf);
     return 0;
 }
@@ -2063,9 +2088,6 @@ int prefill_f16(q3t_dev * c, int n, int n_past) {
                            qkvd, qd, kd, L.k_norm, g.rms_eps, (const float *) c->rope_cos, (const float *) c->rope_sin,
                            kc, vc, c->n_ctx, n_past, c->kv_bf16 ? 1 : 0);
         if (pf_attention(c, L, kc, vc, n, n_past, true)) return -1;
-        const size_t na = (size_t) n * qd;
-        hipLaunchKernelGGL(pf::k_rows_h16, dim3((unsigned) std::min<size_t>((na + kBlock - 1) / kBlock, 4096)),
-                           dim3(kBlock), 0, c->stream, (const float *) c->pf_att, qd, qd, n, c->pf_h);
         pf_gemm_h16(c, L.wo, d, qd, n, c->pf_h, nullptr, qd, nullptr, c->pf_xb, x, d);
         hipLaunchKernelGGL(pf::k_rmsnorm_rows_h16, dim3(n), dim3(kBlock), 0, c->stream, (const float *) c->pf_xb,
                            L.ffn_norm, g.rms_eps, d, c->pf_h);

@@ -866,15 +866,14 @@ constexpr int kVS = 72;          // LDS row stride (halves) of staged P and V^T 
 
 __device__ __forceinline__ double kvd(uint16_t h, bool bf) { return (double) kv2f(h, bf); }
 
-// grid (n, ceil(n_head / 4)), one wave per (row, head): q of row r, head h
-// (QK-norm, NEOX RoPE at position n_past + r) rounded to the cache type, into
-// Qh[h][r][128].
-__global__ __launch_bounds__(kBlock) void k_att_q(const float * __restrict__ qkv, int32_t qkv_stride,
-                                                  const float * __restrict__ q_norm, float eps,
-                                                  const float * __restrict__ rc, const float * __restrict__ rs,
-                                                  int32_t n, int32_t n_past, int32_t n_head, uint16_t * __restrict__ Qh,
-                                                  int32_t bf) {
-    const int row = blockIdx.x, h = blockIdx.y * 4 + (threadIdx.x >> 6), l = threadIdx.x & 63, pos = n_past + row;
+// One wave per (row, head), heads 4 hq .. 4 hq + 3 of a row in a workgroup: q of
+// row r, head h (QK-norm, NEOX RoPE at position n_past + r) rounded to the cache
+// type, into Qh[h][r][128].
+__device__ __forceinline__ void att_q_rows(const float * __restrict__ qkv, int32_t qkv_stride,
+                                           const float * __restrict__ q_norm, float eps, const float * __restrict__ rc,
+                                           const float * __restrict__ rs, int32_t n, int32_t n_past, int32_t n_head,
+                                           uint16_t * __restrict__ Qh, int32_t bf, int row, int hq) {
+    const int h = hq * 4 + (threadIdx.x >> 6), l = threadIdx.x & 63, pos = n_past + row;
     if (h >= n_head) return;                      // whole wave; no workgroup barrier follows
     const float * src = qkv + (size_t) row * qkv_stride + h * kHD;
     float x0 = src[l], x1 = src[64 + l];
@@ -882,6 +881,15 @@ __global__ __launch_bounds__(kBlock) void k_att_q(const float * __restrict__ qkv
     uint16_t * dst = Qh + ((size_t) h * n + row) * kHD;
     dst[l] = f2kv(x0, bf);
     dst[64 + l] = f2kv(x1, bf);
+}
+
+// grid (n, ceil(n_head / 4))
+__global__ __launch_bounds__(kBlock) void k_att_q(const float * __restrict__ qkv, int32_t qkv_stride,
+                                                  const float * __restrict__ q_norm, float eps,
+                                                  const float * __restrict__ rc, const float * __restrict__ rs,
+                                                  int32_t n, int32_t n_past, int32_t n_head, uint16_t * __restrict__ Qh,
+                                                  int32_t bf) {
+    att_q_rows(qkv, qkv_stride, q_norm, eps, rc, rs, n, n_past, n_head, Qh, bf, blockIdx.x, blockIdx.y);
 }
 
 // grid (n_head, Y, 2): workgroup y takes 64-row tiles y and tiles - 1 - y, so
@@ -900,30 +908,6 @@ __global__ __launch_bounds__(kBlock) void k_att_q(const float * __restrict__ qkv
 // registers while tile s's MFMAs run; rows past the tile's last position
 // staged as zero).
 constexpr int kAttT = 256;       // threads of the MFMA attention kernels
-
-// One 16x16x32 MFMA with fp32 accumulation on fp16 (or, bf, bfloat16)
-// operands held as 16-bit patterns: the fast forms of the attention kernels.
-template <bool BF>
-__device__ __forceinline__ f4v mfma_h32(const int4 & a, const int4 & b, f4v c) {
-    const v4i av = (v4i){a.x, a.y, a.z, a.w}, bv = (v4i){b.x, b.y, b.z, b.w};
-    if constexpr (BF) {
-        typedef __bf16 b8v __attribute__((ext_vector_type(8)));
-        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(b8v, av), __builtin_bit_cast(b8v, bv), c, 0, 0, 0);
-    } else {
-        return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8v, av), __builtin_bit_cast(h8v, bv), c, 0, 0, 0);
-    }
-}
-
-// FAST: the scores of a step on 16x16x32 fp16 (bfloat16) MFMAs with fp32
-// accumulation (the reference's F16 K.Q product class) instead of the exact
-// f64 MFMA sums: lane (i, k) supplies dims 32c + 8k .. +7 of q row 16w + i as
-// A and of position 16 t4 + i as B for MFMA c of 4, and its accumulator
-// element r is row 16w + 4k + r, position 16 t4 + i.
-__global__ __launch_bounds__(kAttT) void k_att_scores_fast(const uint16_t * __restrict__ Qh,
-                                                            const uint16_t * __restrict__ kc, int32_t n_ctx,
-                                                            int32_t n_head, int32_t n_kv_head, int32_t n,
-                                                            int32_t n_past, float scale, float * __restrict__ S,
-                                                            int32_t ls, int32_t bf);
 
 __device__ __forceinline__ void att_scores_body(const uint16_t * __restrict__ Qh, const uint16_t * __restrict__ kc,
                                                 int32_t n_ctx, int32_t n_head, int32_t n_kv_head, int32_t n,
@@ -1018,90 +1002,6 @@ __global__ __launch_bounds__(kAttT) void k_att_scores(const uint16_t * __restric
                                                        float * __restrict__ S, int32_t ls, int32_t bf) {
     __shared__ __align__(16) uint16_t kt[2][kAT * kKS];
     att_scores_body(Qh, kc, n_ctx, n_head, n_kv_head, n, n_past, scale, S, ls, bf, kt);
-}
-
-// The fast form of k_att_scores (see its declaration); same grid, tile
-// pairing, K staging and masking.
-template <bool BF>
-__device__ __forceinline__ void att_scores_fast_body(const uint16_t * __restrict__ Qh, const uint16_t * __restrict__ kc,
-                                                     int32_t n_ctx, int32_t n_head, int32_t n_kv_head, int32_t n,
-                                                     int32_t n_past, float scale, float * __restrict__ S, int32_t ls,
-                                                     uint16_t (*kt)[kAT * kKS]) {
-    const int h = blockIdx.x, tiles = (n + kAT - 1) / kAT, g = h / (n_head / n_kv_head), grp = blockIdx.z;
-    const int t = threadIdx.x, w = t >> 6, l = t & 63, i = l & 15, k = l >> 4;
-    const int krow = t >> 4, kch = t & 15;
-    const uint16_t * kbase = kc + (size_t) g * n_ctx * kHD + 8 * kch;
-    const int y = blockIdx.y, Y = gridDim.y;
-    const bool spread = 2 * Y + 1 == tiles;
-    for (int pass = 0; pass < (spread ? 3 : 2); ++pass) {
-        const int tile = pass == 0 ? y : pass == 1 ? tiles - 1 - y : Y;
-        if (pass == 1 && tile == y) break;
-        const int row0 = tile * kAT, my_row = row0 + 16 * w + i;
-        const int lim_tile = n_past + min(row0 + kAT, n) - 1;
-        if (lim_tile < 64 * grp) continue;
-        const int nst = (lim_tile - 64 * grp) / (2 * kAT) + 1;
-        const int st0 = pass == 2 ? y : 0, sd = pass == 2 ? Y : 1;
-        if (st0 >= nst) continue;
-        int4 qa[4];                                             // dims 32c + 8k .. +7 of row my_row
-        {
-            const bool ok = my_row < n;
-            const int4 * src = (const int4 *) (Qh + ((size_t) h * n + (ok ? my_row : 0)) * kHD + 8 * k);
-#pragma unroll
-            for (int c = 0; c < 4; ++c) qa[c] = ok ? src[4 * c] : make_int4(0, 0, 0, 0);
-        }
-        int4 rk[4];
-        int kok[4];
-        auto fetch = [&](int j0) {
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const int j = j0 + krow + 16 * u;
-                kok[u] = j <= lim_tile;
-                rk[u] = *(const int4 *) (kbase + (size_t) min(j, lim_tile) * kHD);
-            }
-        };
-        auto stash = [&](int buf) {
-#pragma unroll
-            for (int u = 0; u < 4; ++u)
-                *(int4 *) (&kt[buf][(krow + 16 * u) * kKS + 8 * kch]) = kok[u] ? rk[u] : make_int4(0, 0, 0, 0);
-        };
-        fetch(2 * kAT * st0 + 64 * grp);
-        stash(0);
-        __syncthreads();
-        for (int st = st0, it = 0; st < nst; st += sd, ++it) {
-            const int buf = it & 1, j0 = 2 * kAT * st + 64 * grp;
-            const bool more = st + sd < nst;
-            if (more) fetch(j0 + 2 * kAT * sd);
-            f4v acc[4];
-#pragma unroll
-            for (int t4 = 0; t4 < 4; ++t4) acc[t4] = (f4v){0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int c = 0; c < 4; ++c)
-#pragma unroll
-                for (int t4 = 0; t4 < 4; ++t4)
-                    acc[t4] = mfma_h32<BF>(qa[c], *(const int4 *) (&kt[buf][(16 * t4 + i) * kKS + 32 * c + 8 * k]),
-                                           acc[t4]);
-#pragma unroll
-            for (int t4 = 0; t4 < 4; ++t4)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int row = row0 + 16 * w + 4 * k + r, j = j0 + 16 * t4 + i;
-                    if (row < n && j <= n_past + row) S[((size_t) h * n + row) * ls + j] = acc[t4][r] * scale;
-                }
-            __asm__ volatile("" ::: "memory");
-            if (more) stash(buf ^ 1);
-            __syncthreads();
-        }
-    }
-}
-
-__global__ __launch_bounds__(kAttT) void k_att_scores_fast(const uint16_t * __restrict__ Qh,
-                                                            const uint16_t * __restrict__ kc, int32_t n_ctx,
-                                                            int32_t n_head, int32_t n_kv_head, int32_t n,
-                                                            int32_t n_past, float scale, float * __restrict__ S,
-                                                            int32_t ls, int32_t bf) {
-    __shared__ __align__(16) uint16_t kt[2][kAT * kKS];
-    if (bf) att_scores_fast_body<true>(Qh, kc, n_ctx, n_head, n_kv_head, n, n_past, scale, S, ls, kt);
-    else att_scores_fast_body<false>(Qh, kc, n_ctx, n_head, n_kv_head, n, n_past, scale, S, ls, kt);
 }
 
 // One row held in registers, R positions per lane (cnt <= 64 R).  Each lane
@@ -1292,121 +1192,6 @@ __global__ __launch_bounds__(kAttT, 4) void k_att_pv(const uint16_t * __restrict
     __shared__ __align__(16) uint16_t pt[2][kAT * kVS];      // [row][position]
     __shared__ __align__(16) uint16_t vt[2][kAT * kVN];      // [position][dim - 64 grp]
     att_pv_body(P, ls, vc, n_ctx, n_head, n_kv_head, n, n_past, out, out_stride, bf, pt, vt);
-}
-
-// The fast form of k_att_pv: P.V on 16x16x32 fp16 (bfloat16) MFMAs with
-// fp32 accumulation.  Same grid, tile pairing, P staging and masks; the V
-// tile is staged transposed ([dim][position], 8 two-byte stores per 8-dim
-// chunk) so that lane (i, k) reads positions 32q + 8k .. +7 of dim 16 b + i as
-// one 16-byte B operand, against P row 16w + i (A).  Accumulator b holds dims
-// 64 grp + 16 b + i of rows 16w + 4k + r (the middle-tile row groups: wave w's
-// dims 16 w + i of rows 16 rg + 4k + r).
-constexpr int kVT = 64 + 8;      // LDS row stride (halves) of the transposed V tile
-template <bool BF>
-__device__ __forceinline__ void att_pv_fast_body(const uint16_t * __restrict__ P, int32_t ls,
-                                                 const uint16_t * __restrict__ vc, int32_t n_ctx, int32_t n_head,
-                                                 int32_t n_kv_head, int32_t n, int32_t n_past, float * __restrict__ out,
-                                                 int32_t out_stride, uint16_t (*pt)[kAT * kVS],
-                                                 uint16_t (*vt)[kAT * kVT]) {
-    const int h = blockIdx.x, tiles = (n + kAT - 1) / kAT, g = h / (n_head / n_kv_head), grp = blockIdx.z;
-    const int t = threadIdx.x, w = t >> 6, l = t & 63, i = l & 15, k = l >> 4;
-    const int srow = t >> 3, sch = t & 7;
-    const uint16_t * vbase = vc + (size_t) g * n_ctx * kHD + 64 * grp + 8 * sch;
-    const int y = blockIdx.y, Y = gridDim.y;
-    const int nrg = (2 * Y + 1 == tiles && y < 4) ? (4 - y + Y - 1) / Y : 0;
-  for (int pass = 0; pass < 2 + nrg; ++pass) {
-    const int rg = pass < 2 ? -1 : y + (pass - 2) * Y;
-    const int tile = pass == 0 ? y : pass == 1 ? tiles - 1 - y : Y;
-    if (pass == 1 && tile == y) continue;
-    const int row0 = tile * kAT, prow = rg < 0 ? 16 * w : 16 * rg;
-    const int lim_tile = n_past + min(row0 + kAT, n) - 1;
-    const int nst = lim_tile / kAT + 1;
-    int plim[2];
-    const uint16_t * prp[2];
-#pragma unroll
-    for (int u = 0; u < 2; ++u) {
-        const int prw = row0 + srow + 32 * u;
-        plim[u] = prw < n ? n_past + prw : -1;
-        prp[u] = P + ((size_t) h * n + (prw < n ? prw : 0)) * ls + 8 * sch;
-    }
-    int4 rp[2], rv[2];
-    int pvalid[2], vok[2];
-    auto fetch = [&](int j0) {
-#pragma unroll
-        for (int u = 0; u < 2; ++u) {
-            pvalid[u] = min(max(plim[u] - (j0 + 8 * sch) + 1, 0), 8);
-            rp[u] = *(const int4 *) (prp[u] + (pvalid[u] > 0 ? j0 : 0));
-            const int pos = j0 + srow + 32 * u;
-            vok[u] = pos <= lim_tile;
-            rv[u] = *(const int4 *) (vbase + (size_t) min(pos, lim_tile) * kHD);
-        }
-    };
-    auto stash = [&](int buf) {
-#pragma unroll
-        for (int u = 0; u < 2; ++u) {
-            int4 v = rp[u];
-            const int pv = pvalid[u];
-            if (pv < 8) {
-                const auto m = [pv](int e) { return (2 * e < pv ? 0xffff : 0) | (2 * e + 1 < pv ? (int) 0xffff0000u : 0); };
-                v.x &= m(0); v.y &= m(1); v.z &= m(2); v.w &= m(3);
-            }
-            *(int4 *) (&pt[buf][(srow + 32 * u) * kVS + 8 * sch]) = v;
-            const int4 vv = vok[u] ? rv[u] : make_int4(0, 0, 0, 0);
-            const int pos = srow + 32 * u;
-#pragma unroll
-            for (int e = 0; e < 8; ++e) vt[buf][(8 * sch + e) * kVT + pos] = h8bits(vv, e);
-        }
-    };
-    f4v acc[4];
-#pragma unroll
-    for (int b = 0; b < 4; ++b) acc[b] = (f4v){0.f, 0.f, 0.f, 0.f};
-    fetch(0);
-    stash(0);
-    __syncthreads();
-    for (int st = 0; st < nst; ++st) {
-        const int buf = st & 1;
-        if (st + 1 < nst) fetch((st + 1) * kAT);
-#pragma unroll
-        for (int q = 0; q < 2; ++q) {
-            const int4 pa = *(const int4 *) (&pt[buf][(prow + i) * kVS + 32 * q + 8 * k]);
-            if (rg < 0) {
-#pragma unroll
-                for (int b = 0; b < 4; ++b)
-                    acc[b] = mfma_h32<BF>(pa, *(const int4 *) (&vt[buf][(16 * b + i) * kVT + 32 * q + 8 * k]), acc[b]);
-            } else {
-                acc[0] = mfma_h32<BF>(pa, *(const int4 *) (&vt[buf][(16 * w + i) * kVT + 32 * q + 8 * k]), acc[0]);
-            }
-        }
-        __asm__ volatile("" ::: "memory");
-        if (st + 1 < nst) stash(buf ^ 1);
-        __syncthreads();
-    }
-    if (rg < 0) {
-#pragma unroll
-        for (int b = 0; b < 4; ++b)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int row = row0 + 16 * w + 4 * k + r;
-                if (row < n) out[(size_t) row * out_stride + h * kHD + 64 * grp + 16 * b + i] = acc[b][r];
-            }
-    } else {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int row = row0 + 16 * rg + 4 * k + r;
-            if (row < n) out[(size_t) row * out_stride + h * kHD + 64 * grp + 16 * w + i] = acc[0][r];
-        }
-    }
-  }
-}
-
-__global__ __launch_bounds__(kAttT, 4) void k_att_pv_fast(const uint16_t * __restrict__ P, int32_t ls,
-                                                        const uint16_t * __restrict__ vc, int32_t n_ctx,
-                                                        int32_t n_head, int32_t n_kv_head, int32_t n, int32_t n_past,
-                                                        float * __restrict__ out, int32_t out_stride, int32_t bf) {
-    __shared__ __align__(16) uint16_t pt[2][kAT * kVS];
-    __shared__ __align__(16) uint16_t vt[2][kAT * kVT];
-    if (bf) att_pv_fast_body<true>(P, ls, vc, n_ctx, n_head, n_kv_head, n, n_past, out, out_stride, pt, vt);
-    else att_pv_fast_body<false>(P, ls, vc, n_ctx, n_head, n_kv_head, n, n_past, out, out_stride, pt, vt);
 }
 
 __host__ __device__ constexpr size_t attn_rows_lds_bytes(int n_ctx) {

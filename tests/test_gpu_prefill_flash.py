@@ -1,0 +1,65 @@
+"""The fast attention of the tiled F16 prefill (scores, softmax and P.V in one kernel).
+
+Its rows against the exact form's (Q3T_PF_EXACT=1) over the edges of the 64-row and 64-position tiles, behind
+cached positions whose keys grow or shrink with the position, so that the running maximum rises in every tile or
+never again, and with a bfloat16 cache.  Tolerance: the probabilities are rounded to 11 bits (bfloat16: 8), each
+GEMM input to 11, so a row moves by a few 2^-12 (2^-9) of its largest value per layer; two layers, with room for
+the sums' own spread, stay within 2^-8 (2^-6).  The second layer's q comes from sums that the two forms round
+differently, and a q element that falls the other way moves by 2^-10 (2^-7) of itself: against the grown keys (up
+to 30, q up to 3, scale 2^-3.5) a score then moves by 30 * 3 * 2^-3.5 * 2^-10 = 2^-7 (2^-4), and the weight it carries
+by as much; those rows get twice the tolerance.
+"""
+import sys
+
+import numpy as np
+import pytest
+import torch
+
+from qwen3_tts_amd import config as qcfg
+from qwen3_tts_amd.device import Device
+from qwen3_tts_amd.synth import Weights
+
+pytestmark = pytest.mark.gpu
+BF16 = 30
+
+
+def say(*a):
+    print(*a, file=sys.stderr, flush=True)
+
+
+@pytest.fixture(scope="module", params=["f16", "bf16"])
+def model(request):
+    cfg = qcfg.tiny()
+    dev = Device(cfg)
+    dev.upload_weights(Weights(cfg, "f16", seed=31))
+    if request.param == "bf16":
+        dev.kv_set_type(BF16)
+    yield cfg, dev, request.param == "bf16"
+    dev.close()
+
+
+SIZES = [(0, 64), (0, 65), (0, 127), (0, 193), (1, 64), (63, 65), (10, 119), (300, 321), (3000, 70)]
+
+
+@pytest.mark.parametrize("past,n,growth", [(p, n, g) for p, n in SIZES for g in (0.0, 2.0, -2.0) if p or not g])
+def test_flash_attention_against_exact(model, monkeypatch, past, n, growth):
+    cfg, dev, bf = model
+    dev.kv_reserve(past + n)
+    rng = np.random.default_rng(past + n)
+    for layer in range(cfg.n_layers if past else 0):
+        kv = rng.standard_normal((2, past, cfg.n_kv_head, cfg.head_dim)).astype(np.float32)
+        kv[0] *= np.exp(growth * np.linspace(-1, 1, past))[:, None, None]
+        if bf:
+            k, v = (torch.from_numpy(a).bfloat16().view(torch.int16).numpy().view(np.uint16) for a in kv)
+        else:
+            k, v = kv.astype(np.float16)
+        dev.kv_write(layer, k, v)
+    rows = (rng.standard_normal((n, cfg.hidden_size)) * 0.05).astype(np.float32)
+    out = {}
+    for exact in ("1", "0"):
+        monkeypatch.setenv("Q3T_PF_EXACT", exact)
+        out[exact] = dev.prefill(rows, past)[0].astype(np.float64)
+    rel = np.abs(out["0"] - out["1"]).max(axis=1) / np.abs(out["1"]).max(axis=1)
+    say(f"[gpu] fast attention, {n} rows at {past}, growth {growth}, bf16 {bf}: rel max {rel.max():.2e}")
+    assert rel.max() > 0          # the fast form ran
+    assert rel.max() <= (2.0**-6 if bf else 2.0**-8) * (2 if growth else 1)
