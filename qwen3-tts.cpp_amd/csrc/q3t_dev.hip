@@ -1907,23 +1907,26 @@ void pf_gemm_f16(q3t_dev * c, const Slot & w, int N, int K, int n, const float *
 }
 
 // F16 weights x fp16 rows on the fast fp16-MFMA GEMM (fp32 accumulation):
-// y = (W . xh[t] (+ W . xl[t])) * xsc[t] (+ res).  128 x 128 tiles with one
-// stage in flight when that gives at least one workgroup per CU, else
-// 128 x 64 tiles with two stages in flight (and always for the two-plane
-// input); measured best on the 0.6B shapes at 2,048 rows: QKV 30 us, Wo 27 us,
-// gate / up 29 us, the two-plane down 47 us.
+// y = (W . xh[t] (+ W . xl[t])) * xsc[t] (+ res).  The largest tile that still
+// gives the card enough workgroups, 0.6B shapes, us (QKV, gate, Wo, two-plane down):
+//   128 x 128, 2 stages in flight, from one workgroup a CU on: 2,049 rows 34, 25
+//     (64 x 64: 36, 30); below that 600 rows 16, 16 against 15, 12;
+//   128 x 64, 2 stages, the two-plane input from one workgroup a CU on: 2,049 rows
+//     down 56 (64 x 64: 60);
+//   64 x 64, 4 stages, from half a workgroup a CU on: 2,049 rows Wo 24 (128 x 64: 26),
+//     600 rows Wo 13, down 25, 200 rows QKV 8 (32 x 32: 11);
+//   32 x 32, 4 stages, below: 200 rows Wo 9, down 14 (64 x 64: 13, 24).
+// K is a multiple of 256 (four stages), as pf_f16_fast checks.
 void pf_gemm_h16(q3t_dev * c, const Slot & w, int N, int K, int n, const uint16_t * xh, const uint16_t * xl, int xs,
                  const float * xsc, float * y, const float * res, int rs) {
-    constexpr int BR = 32 * 4;
-    const bool big = !xl && (int64_t) (N / BR) * ((n + 127) / 128) >= c->n_cu;
-    const int TT = big ? 4 : 2;
-    const dim3 grid(N / BR, (n + 32 * TT - 1) / (32 * TT));
-#define Q3T_PF_H16(tt, lo, pd)                                                                                    \
-    hipLaunchKernelGGL((pf::k_gemm_h16<4, tt, lo, pd>), grid, dim3(kBlock), 0, c->stream, (const uint16_t *) w.data, \
-                       K, xh, xl, xs, xsc, n, y, N, res, rs)
-    if (xl) Q3T_PF_H16(2, true, 2);
-    else if (big) Q3T_PF_H16(4, false, 1);
-    else Q3T_PF_H16(2, false, 2);
+    const auto tiles = [&](int wm, int tt) { return (int64_t) (N / (32 * wm)) * ((n + 32 * tt - 1) / (32 * tt)); };
+#define Q3T_PF_H16(wm, tt, lo, pd)                                                                                \
+    hipLaunchKernelGGL((pf::k_gemm_h16<wm, tt, lo, pd>), dim3(N / (32 * wm), (n + 32 * tt - 1) / (32 * tt)),       \
+                       dim3(kBlock), 0, c->stream, (const uint16_t *) w.data, K, xh, xl, xs, xsc, n, y, N, res, rs)
+    if (!xl && tiles(4, 4) >= c->n_cu) Q3T_PF_H16(4, 4, false, 2);
+    else if (xl && tiles(4, 2) >= c->n_cu) Q3T_PF_H16(4, 2, true, 2);
+    else if (2 * tiles(2, 2) >= c->n_cu) { if (xl) Q3T_PF_H16(2, 2, true, 4); else Q3T_PF_H16(2, 2, false, 4); }
+    else { if (xl) Q3T_PF_H16(1, 1, true, 4); else Q3T_PF_H16(1, 1, false, 4); }
 #undef Q3T_PF_H16
 }
 
@@ -1943,7 +1946,7 @@ bool pf_exact() {
 bool pf_f16_fast(const q3t_config & g) {
     if (pf_exact()) return false;
     const int d = g.hidden_size, qd = g.n_head * g.head_dim, qkvd = qd + 2 * g.n_kv_head * g.head_dim;
-    return d % 128 == 0 && qkvd % 128 == 0 && g.ffn_size % 128 == 0 && qd % pf::kHK == 0 && d % pf::kHK == 0 &&
+    return d % 256 == 0 && qkvd % 128 == 0 && g.ffn_size % 256 == 0 && qd % 256 == 0 &&
            g.ffn_size <= 16 * kBlock;
 }
 

@@ -514,20 +514,27 @@ __global__ __launch_bounds__(kBlock) void k_gemm_f16(const uint16_t * __restrict
 //     one float4 store;
 //   - K in stages of 64 staged in LDS as 16-byte chunks, chunk c of row r at
 //     position c ^ (r & 7) (8 consecutive rows of one chunk hit distinct
-//     banks), double-buffered: stage s + 1's global loads are in flight
-//     during stage s's MFMAs;
+//     banks), double-buffered, the global loads of PD later stages in flight;
 //   - tokens past n stage zeros and store nothing.
-// Requires N % (32 WM) == 0 and K % 64 == 0 (the host checks).
+// Requires N % (32 WM) == 0 and K % (64 PD) == 0 (the host checks).
 typedef _Float16 h8v __attribute__((ext_vector_type(8)));
 typedef float f4v __attribute__((ext_vector_type(4)));
 constexpr int kHK = 64;            // K per stage (8 chunks of 8 halves)
 
 __device__ __forceinline__ int hswz(int r, int c) { return r * kHK + ((c ^ (r & 7)) << 3); }
 
+// f(0), ..., f(M - 1) with compile-time constants
+template <int M, typename F>
+__device__ __forceinline__ void each(F && f) {
+    if constexpr (M > 0) {
+        each<M - 1>(f);
+        f(std::integral_constant<int, M - 1>{});
+    }
+}
+
 // WM: 16-row MFMA tiles per wave along the weight rows (workgroup rows 32 WM);
 // TT: 16-token tiles per wave (workgroup tokens 32 TT); LO: the low plane;
-// PD: stages in flight (1: the next stage's loads overlap this stage's
-// MFMAs; 2: two register sets, loads issued two stages ahead).
+// PD: stages in flight, one register set each; K % (64 PD) == 0.
 template <int WM, int TT, bool LO, int PD>
 struct H16Tile {
     static constexpr int BR = 32 * WM, BT = 32 * TT;         // workgroup tile
@@ -629,31 +636,29 @@ __global__ __launch_bounds__(kBlock) void k_gemm_h16(const uint16_t * __restrict
         __asm__ volatile("" ::: "memory");
         __builtin_amdgcn_sched_barrier(0);
     };
-    using C0 = std::integral_constant<int, 0>;
-    using C1 = std::integral_constant<int, PD == 2 ? 1 : 0>;
+    // Stage s waits in register set s % PD and is computed from LDS buffer s & 1.
+    // Step s issues stage s + PD's loads, runs stage s's MFMAs, then stashes stage
+    // s + 1.  No load or stash of the main loop is under a condition: behind a
+    // branch the compiler waits for every load in flight (with the branch a stage of a
+    // lone workgroup took a whole load's latency, 1.05 us: down at 200 rows 50 us, now 14).
     const int S = K / kHK;
-    // stage s computes from LDS buffer s & 1.  PD 1: stage s + 1 is loaded into
-    // the one register set during stage s and stashed after its MFMAs.  PD 2:
-    // stage s + 2 is loaded into set s & 1 during stage s, while stage s + 1
-    // (set (s + 1) & 1, loaded during stage s - 1) is stashed after the MFMAs.
-    auto step = [&](int s, auto cur, auto nxt) {
-        if (PD == 1 && s + 1 < S) fetch(C0{}, (s + 1) * kHK);
-        if (PD == 2 && s + 2 < S) fetch(cur, (s + 2) * kHK);
-        mfmas(s & 1);
-        if (s + 1 < S) {
-            if (PD == 1) stash(C0{}, (s + 1) & 1);
-            else stash(nxt, (s + 1) & 1);
+    auto step = [&](int s, auto j_c, auto more_c, auto last_c) {
+        constexpr int j = decltype(j_c)::value;
+        if constexpr (decltype(more_c)::value) fetch(std::integral_constant<int, j>{}, (s + j + PD) * kHK);
+        mfmas((s + j) & 1);
+        if constexpr (!decltype(last_c)::value) {
+            stash(std::integral_constant<int, (j + 1) % PD>{}, (s + j + 1) & 1);
+            __syncthreads();
         }
-        __syncthreads();
     };
-    fetch(C0{}, 0);
-    stash(C0{}, 0);
-    if (PD == 2 && S > 1) fetch(C1{}, kHK);
+    using On = std::true_type;
+    using Off = std::false_type;
+    each<PD>([&](auto j) { fetch(j, decltype(j)::value * kHK); });
+    stash(std::integral_constant<int, 0>{}, 0);
     __syncthreads();
-    for (int s = 0; s < S; s += 2) {
-        step(s, C0{}, C1{});
-        if (s + 1 < S) step(s + 1, C1{}, C0{});
-    }
+    for (int s = 0; s < S - PD; s += PD) each<PD>([&](auto j) { step(s, j, On{}, Off{}); });
+    each<PD - 1>([&](auto j) { step(S - PD, j, Off{}, Off{}); });
+    step(S - PD, std::integral_constant<int, PD - 1>{}, Off{}, On{});
 #pragma unroll
     for (int j = 0; j < TT; ++j) {
         const int tok = t0 + wt * 16 * TT + 16 * j + lm;

@@ -1,4 +1,4 @@
-"""The fast attention of the tiled F16 prefill (scores, softmax and P.V in one kernel).
+"""The fast attention of the tiled F16 prefill (scores, softmax and P.V in one kernel) and its GEMM tiles.
 
 Its rows against the exact form's (Q3T_PF_EXACT=1) over the edges of the 64-row and 64-position tiles, behind
 cached positions whose keys grow or shrink with the position, so that the running maximum rises in every tile or
@@ -63,3 +63,27 @@ def test_flash_attention_against_exact(model, monkeypatch, past, n, growth):
     say(f"[gpu] fast attention, {n} rows at {past}, growth {growth}, bf16 {bf}: rel max {rel.max():.2e}")
     assert rel.max() > 0          # the fast form ran
     assert rel.max() <= (2.0**-6 if bf else 2.0**-8) * (2 if growth else 1)
+
+
+@pytest.mark.parametrize("n", [40, 65, 200, 600, 2049])
+@pytest.mark.parametrize("hidden,ffn", [(256, 512), (1024, 3072)])
+def test_fast_gemm_tiles_against_exact(monkeypatch, hidden, ffn, n):
+    """The fast GEMM's tiles and stage counts: the shortest K (four stages, all in flight at once), rows
+    below and past a tile, few and many workgroups.  Every input is rounded to 11 bits and summed in fp32, in the same order
+    whatever the tile: the bound of the fp16 rows above."""
+    cfg = qcfg.tiny(hidden=hidden, ffn=ffn, n_layers=1)
+    monkeypatch.setenv("Q3T_PREFILL_MFMA", "1")
+    dev = Device(cfg)
+    try:
+        dev.upload_weights(Weights(cfg, "f16", seed=37))
+        dev.kv_reserve(n)
+        rows = (np.random.default_rng(n).standard_normal((n, hidden)) * 0.05).astype(np.float32)
+        out = {}
+        for exact in ("1", "0"):
+            monkeypatch.setenv("Q3T_PF_EXACT", exact)
+            out[exact] = dev.prefill(rows, 0)[0].astype(np.float64)
+    finally:
+        dev.close()
+    rel = np.abs(out["0"] - out["1"]).max(axis=1) / np.abs(out["1"]).max(axis=1)
+    say(f"[gpu] fast GEMM tiles, {n} rows of {hidden}, {ffn}: rel max {rel.max():.2e}")
+    assert 0 < rel.max() <= 2.0**-8
