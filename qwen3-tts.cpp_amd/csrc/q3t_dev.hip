@@ -2009,11 +2009,12 @@ int pf_attention(q3t_dev * c, const LayerDev & L, const uint16_t * kc, const uin
         a.qkv = c->pf_qkv; a.qkv_stride = qkvd; a.q_norm = L.q_norm; a.eps = g.rms_eps;
         a.rc = c->rope_cos; a.rs = c->rope_sin; a.kc = kc; a.vc = vc;
         a.n_ctx = c->n_ctx; a.n_head = g.n_head; a.n_kv_head = g.n_kv_head; a.n = n; a.n_past = n_past; a.bf = bf;
+        a.batch = std::max(1, c->n_cu / g.n_head);
         a.Qh = (uint16_t *) c->pf_dig; a.Vt = a.Qh + qb;
         hipLaunchKernelGGL(pf::k_att_flash_in, dim3((unsigned) (n * ((g.n_head + 3) / 4) + g.n_kv_head * (ls / 64))),
                            dim3(kBlock), 0, c->stream, a);
         hipLaunchKernelGGL(pf::k_att_flash, dim3(g.n_head, (n + pf::kAT - 1) / pf::kAT), dim3(pf::kFT), 0, c->stream, a,
-                           scale * 1.44269504088896341f, c->pf_h, qd);
+                           scale, c->pf_h, qd);
         return 0;
     }
     // the probabilities buffer also holds the q rows [n_head][n][128] first

@@ -65,6 +65,46 @@ def test_flash_attention_against_exact(model, monkeypatch, past, n, growth):
     assert rel.max() <= (2.0**-6 if bf else 2.0**-8) * (2 if growth else 1)
 
 
+@pytest.mark.parametrize("kv", ["f16", "bf16"])
+@pytest.mark.parametrize("past,n", [(1, 64), (37, 65), (100, 200), (700, 129), (2900, 100)])
+def test_flash_probabilities_are_normalised_then_rounded(monkeypatch, past, n, kv):
+    """Every score zero (no Q weights), V one in the cache and zero in the new rows: a row of c positions is
+    past * p with p the 16-bit rounding of fp32(1 / c), the sum of c ones taken in full.  The products are
+    whole multiples of p below 2^12, exact in any order, and the output projection copies one attention value
+    to each of the hidden dims 128 .. 255, beside ones in the dims before, so the values come out whole."""
+    monkeypatch.setenv("Q3T_PF_EXACT", "0")
+    cfg = qcfg.tiny(n_layers=1)
+    w = Weights(cfg, "f16", seed=41)
+    blk = "talker.blk.0."
+    for name in ("attn_q", "attn_k", "attn_v", "attn_output", "ffn_down"):
+        w[blk + name + ".weight"][2][:] = 0
+    w["talker.output_norm.weight"][2][:] = 1
+    m = np.arange(128)
+    wo = w[blk + "attn_output.weight"][2].reshape(cfg.hidden_size, cfg.n_head * cfg.head_dim)
+    wo[128 + m, 4 * m + m % 4] = 1
+    dev = Device(cfg)
+    try:
+        dev.upload_weights(w)
+        if kv == "bf16":
+            dev.kv_set_type(BF16)
+        dev.kv_reserve(past + n)
+        shape = (past, cfg.n_kv_head, cfg.head_dim)
+        one = np.uint16(0x3F80) if kv == "bf16" else np.float16(1)
+        dev.kv_write(0, np.zeros(shape, type(one)), np.full(shape, one))
+        rows = np.zeros((n, cfg.hidden_size), np.float32)
+        rows[:, :128] = 1
+        say(f"[gpu] uniform attention, {n} rows at {past}, cache {kv}")
+        hid = dev.prefill(rows, past)[0]
+    finally:
+        dev.close()
+    p = torch.from_numpy((1.0 / np.arange(past + 1, past + n + 1)).astype(np.float32))
+    p = (p.bfloat16() if kv == "bf16" else p.half()).double().numpy()
+    want = (past * p).astype(np.float16)
+    got = (hid[:, 128:] / hid[:, :1]).astype(np.float16)
+    wrong = int((got != want[:, None]).sum())
+    assert wrong == 0, f"{wrong} of {got.size} values"
+
+
 @pytest.mark.parametrize("n", [40, 65, 200, 600, 2049])
 @pytest.mark.parametrize("hidden,ffn", [(256, 512), (1024, 3072)])
 def test_fast_gemm_tiles_against_exact(monkeypatch, hidden, ffn, n):
