@@ -1916,7 +1916,7 @@ void pf_gemm_f16(q3t_dev * c, const Slot & w, int N, int K, int n, const float *
 //   64 x 64, 4 stages, from half a workgroup a CU on: 2,049 rows Wo 24 (128 x 64: 26),
 //     600 rows Wo 13, down 25, 200 rows QKV 8 (32 x 32: 11);
 //   32 x 32, 4 stages, below: 200 rows Wo 9, down 14 (64 x 64: 13, 24).
-// K is a multiple of 256 (four stages), as pf_f16_fast checks.
+// The small tiles hold two stages where K is 128 (Wo of a model with one head): the same sums.
 void pf_gemm_h16(q3t_dev * c, const Slot & w, int N, int K, int n, const uint16_t * xh, const uint16_t * xl, int xs,
                  const float * xsc, float * y, const float * res, int rs) {
     const auto tiles = [&](int wm, int tt) { return (int64_t) (N / (32 * wm)) * ((n + 32 * tt - 1) / (32 * tt)); };
@@ -1925,8 +1925,15 @@ void pf_gemm_h16(q3t_dev * c, const Slot & w, int N, int K, int n, const uint16_
                        dim3(kBlock), 0, c->stream, (const uint16_t *) w.data, K, xh, xl, xs, xsc, n, y, N, res, rs)
     if (!xl && tiles(4, 4) >= c->n_cu) Q3T_PF_H16(4, 4, false, 2);
     else if (xl && tiles(4, 2) >= c->n_cu) Q3T_PF_H16(4, 2, true, 2);
-    else if (2 * tiles(2, 2) >= c->n_cu) { if (xl) Q3T_PF_H16(2, 2, true, 4); else Q3T_PF_H16(2, 2, false, 4); }
-    else { if (xl) Q3T_PF_H16(1, 1, true, 4); else Q3T_PF_H16(1, 1, false, 4); }
+    else if (2 * tiles(2, 2) >= c->n_cu) {
+        if (xl) Q3T_PF_H16(2, 2, true, 4);
+        else if (K % 256) Q3T_PF_H16(2, 2, false, 2);
+        else Q3T_PF_H16(2, 2, false, 4);
+    } else {
+        if (xl) Q3T_PF_H16(1, 1, true, 4);
+        else if (K % 256) Q3T_PF_H16(1, 1, false, 2);
+        else Q3T_PF_H16(1, 1, false, 4);
+    }
 #undef Q3T_PF_H16
 }
 
@@ -1946,7 +1953,7 @@ bool pf_exact() {
 bool pf_f16_fast(const q3t_config & g) {
     if (pf_exact()) return false;
     const int d = g.hidden_size, qd = g.n_head * g.head_dim, qkvd = qd + 2 * g.n_kv_head * g.head_dim;
-    return d % 256 == 0 && qkvd % 128 == 0 && g.ffn_size % 256 == 0 && qd % 256 == 0 &&
+    return d % 256 == 0 && qkvd % 128 == 0 && g.ffn_size % 256 == 0 && qd % 128 == 0 &&
            g.ffn_size <= 16 * kBlock;
 }
 

@@ -105,6 +105,28 @@ def test_flash_probabilities_are_normalised_then_rounded(monkeypatch, past, n, k
     assert wrong == 0, f"{wrong} of {got.size} values"
 
 
+@pytest.mark.parametrize("n", [65, 1100])
+def test_fast_form_of_one_head(monkeypatch, n):
+    """One head: the output projection's K of 128 is half of the four stages that the small tiles hold
+    otherwise (32 x 32 tiles at 65 rows, 64 x 64 at 1,100); the bound of the fp16 rows above, and the fast
+    form ran."""
+    cfg = qcfg.tiny(hidden=512, n_head=1, n_kv_head=1)
+    dev = Device(cfg)
+    try:
+        dev.upload_weights(Weights(cfg, "f16", seed=43))
+        dev.kv_reserve(n)
+        rows = (np.random.default_rng(n).standard_normal((n, cfg.hidden_size)) * 0.05).astype(np.float32)
+        out = {}
+        for exact in ("1", "0"):
+            monkeypatch.setenv("Q3T_PF_EXACT", exact)
+            say(f"[gpu] one head, {n} rows, exact {exact}")
+            out[exact] = dev.prefill(rows, 0)[0].astype(np.float64)
+    finally:
+        dev.close()
+    rel = np.abs(out["0"] - out["1"]).max(axis=1) / np.abs(out["1"]).max(axis=1)
+    assert 0 < rel.max() <= 2.0**-8, rel.max()
+
+
 @pytest.mark.parametrize("n", [40, 65, 200, 600, 2049])
 @pytest.mark.parametrize("hidden,ffn", [(256, 512), (1024, 3072)])
 def test_fast_gemm_tiles_against_exact(monkeypatch, hidden, ffn, n):
