@@ -1964,14 +1964,21 @@ void pf_rows_h16(q3t_dev * c, const float * x, int K, int n, uint16_t * y) {
                        0, c->stream, x, K, K, n, y);
 }
 
+// The flag of values that have no digits; false when the device has no memory for it.
+bool ensure_wide(q3t_dev * c) {
+    if (c->pf_wide) return true;
+    if (dev_alloc_t(c, &c->pf_wide, 1)) { (void) hipGetLastError(); return false; }
+    // on the context's stream, which does not wait for the null stream: the call's
+    // own kernels set and read the flag
+    if (hipMemsetAsync(c->pf_wide, 0, sizeof(int32_t), c->stream) == hipSuccess) return true;
+    dev_free(c, c->pf_wide);
+    c->pf_wide = nullptr;
+    return false;
+}
+
 // Room for `bytes` of attention operands (the digit planes, or the fast form's q
-// rows and V^T tiles) and the flag of values that have no digits; false when the
-// device has no memory for them.
+// rows and V^T tiles); false when the device has no memory for them.
 bool ensure_operands(q3t_dev * c, size_t bytes) {
-    if (!c->pf_wide) {
-        if (dev_alloc_t(c, &c->pf_wide, 1)) { (void) hipGetLastError(); return false; }
-        if (hipMemset(c->pf_wide, 0, sizeof(int32_t)) != hipSuccess) { dev_free(c, c->pf_wide); c->pf_wide = nullptr; return false; }
-    }
     if (bytes <= c->pf_dig_cap) return true;
     dev_free(c, c->pf_dig);
     c->pf_dig = nullptr; c->pf_dig_cap = 0;
@@ -2045,7 +2052,8 @@ int pf_attention(q3t_dev * c, const LayerDev & L, const uint16_t * kc, const uin
     // scores the digit softmax holds in registers (bfloat16 values span more
     // than four digits); without room for the digits, the f64 forms
     const size_t qb = (size_t) g.n_head * n * 4 * kHD, kb = (size_t) g.n_kv_head * ls * 4 * kHD;
-    if (!bf && n_past + n <= pf::kIntMaxPos && !pf_att_f64() && ensure_operands(c, qb + 2 * kb)) {
+    if (!bf && n_past + n <= pf::kIntMaxPos && !pf_att_f64() && ensure_wide(c) &&
+        ensure_operands(c, qb + 2 * kb)) {
         pf::AttInt a{};
         a.qkv = c->pf_qkv; a.qkv_stride = qkvd; a.q_norm = L.q_norm; a.eps = g.rms_eps;
         a.rc = c->rope_cos; a.rs = c->rope_sin; a.kc = kc; a.vc = vc;

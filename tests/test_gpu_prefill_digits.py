@@ -89,3 +89,27 @@ def test_values_without_digits_take_f64(model, monkeypatch, which, value):
     again = both(dev, rows, past, monkeypatch)
     same(again, "again")
     same([plain[0], again[1]], "plain and again")
+
+
+@pytest.mark.parametrize("value", [-300.0, np.inf])
+def test_values_without_digits_in_a_contexts_first_prefill(model, monkeypatch, value):
+    """The flag of such values is allocated, cleared and set by the first prefill that wants digits."""
+    cfg, _ = model
+    past, n = 70, 130
+    kv = np.random.default_rng(8).standard_normal((2, past, cfg.n_kv_head, cfg.head_dim)).astype(np.float16)
+    kv[0, 33, 0, 5] = value
+    rows = (np.random.default_rng(9).standard_normal((n, cfg.hidden_size)) * 0.05).astype(np.float32)
+    out = []
+    for env in ("0", "1"):
+        monkeypatch.setenv("Q3T_PF_ATT_INT", env)
+        dev = Device(cfg)
+        try:
+            dev.upload_weights(Weights(cfg, "q8_0", seed=29))
+            dev.kv_reserve(past + n)
+            for layer in range(cfg.n_layers):
+                dev.kv_write(layer, kv[0], kv[1])
+            say(f"[gpu] first prefill, k = {value} in the cache, digits {env}")
+            out.append(dev.prefill(rows, past))
+        finally:
+            dev.close()
+    same(out, value)

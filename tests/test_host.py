@@ -3,10 +3,15 @@ repetition-loop truncation (src/tts_transformer.cpp:3225-3254), replayed the
 way the driver applies it after each chunk, and the synthetic-weight specs
 (tensor names/shapes/types of create_tensors, src/tts_transformer.cpp:379-668,
 and the converter's dtype policy, scripts/convert_tts_to_gguf.py:249-324)."""
+import os
+import re
+
 import numpy as np
+import pytest
 
 from qwen3_tts_amd import config
 from qwen3_tts_amd.driver import _rep_loop
+from qwen3_tts_amd.device import PKG_DIR
 from qwen3_tts_amd.synth import F16, F32, Q8_0, tensor_specs
 
 
@@ -108,3 +113,13 @@ def test_bench_refuses_more_than_one_gpu():
                        text=True, timeout=120)
     assert r.returncode == 2
     assert "one GPU" in r.stderr
+
+
+@pytest.mark.parametrize("name", ["q3t_dev.hip"])
+def test_device_buffers_are_cleared_on_the_context_stream(name):
+    """A context's stream is non-blocking: a fill on the null stream is not ordered before the kernels that
+    follow it there."""
+    src = open(os.path.join(PKG_DIR, "csrc", name)).read()
+    assert "hipStreamNonBlocking" in src
+    fills = re.findall(r"\bhipMemset\w*\s*\([^;]*;", src)
+    assert fills and [f for f in fills if not re.search(r"hipMemsetAsync\(.*->stream\)", f, re.S)] == []
