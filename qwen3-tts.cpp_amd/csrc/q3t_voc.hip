@@ -455,12 +455,12 @@ int reserve(q3t_voc * v, int32_t n) {
     rc |= alloc(v, &v->ffn, (size_t) n * F);
     rc |= alloc(v, &v->codes, (size_t) n * c.n_codebooks);
     if (rc) return -1;
-    HIP_OK(hipMemset(v->h[0], 0, hn * 2));
-    HIP_OK(hipMemset(v->h[1], 0, hn * 2));
-    HIP_OK(hipMemset(v->mid, 0, mid * 2));
-    HIP_OK(hipMemset(v->hq, 0, (size_t) n * std::max(H, L) * 2));
-    HIP_OK(hipMemset(v->att, 0, (size_t) n * L * 2));
-    HIP_OK(hipMemset(v->ffn, 0, (size_t) n * F * 2));
+    HIP_OK(hipMemsetAsync(v->h[0], 0, hn * 2, v->stream));
+    HIP_OK(hipMemsetAsync(v->h[1], 0, hn * 2, v->stream));
+    HIP_OK(hipMemsetAsync(v->mid, 0, mid * 2, v->stream));
+    HIP_OK(hipMemsetAsync(v->hq, 0, (size_t) n * std::max(H, L) * 2, v->stream));
+    HIP_OK(hipMemsetAsync(v->att, 0, (size_t) n * L * 2, v->stream));
+    HIP_OK(hipMemsetAsync(v->ffn, 0, (size_t) n * F * 2, v->stream));
     v->xf_n = xf; v->h_n = hn; v->mid_n = mid; v->wide_n = wide; v->audio_n = audio;
     v->cap_frames = n;
     return 0;

@@ -115,7 +115,7 @@ def test_bench_refuses_more_than_one_gpu():
     assert "one GPU" in r.stderr
 
 
-@pytest.mark.parametrize("name", ["q3t_dev.hip"])
+@pytest.mark.parametrize("name", ["q3t_dev.hip", "q3t_voc.hip"])
 def test_device_buffers_are_cleared_on_the_context_stream(name):
     """A context's stream is non-blocking: a fill on the null stream is not ordered before the kernels that
     follow it there."""
