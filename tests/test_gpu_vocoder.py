@@ -20,6 +20,7 @@ and identical results whether codes come from host memory or from the frame
 loop's device rows.
 """
 import ctypes
+import dataclasses
 import sys
 
 import numpy as np
@@ -96,10 +97,9 @@ def test_stages_match_oracle(tiny_voc, n, pos0):
 
 @pytest.mark.parametrize("n", [73, 239, 240, 400])
 def test_pre_transformer_attention_forms(tiny_voc, n):
-    """A pre-transformer layer over n rows at position 19: up to 239 rows at
-    these widths (head width 32) the attention stages each head's q, K and V
-    rows in LDS (four query rows per workgroup), from 240 rows it takes the
-    one-wave-per-row kernel; both within the stage tolerances of the oracle."""
+    """A pre-transformer layer over n rows at position 19, head width 32: K and
+    V in 64-key LDS tiles, two query rows per wave, over two to seven tiles;
+    within the stage tolerances of the oracle."""
     c, w, g, o = tiny_voc
     width = o.stages(codes_for(2, 1), 0)["input_proj"].shape[1]
     x = (np.random.default_rng(n).standard_normal((n, width)) * 0.5).astype(np.float32)
@@ -123,6 +123,42 @@ def test_pre_transformer_attention_forms_agree(tiny_voc):
     want = g.run_stage("pre_tfm.0", x, 5)
     for n in (1, 3, 63, 64, 65, 127, 129, 400, 5000):
         say(f"[gpu] pre_tfm.0 over {n} rows")
+        assert np.array_equal(g.run_stage("pre_tfm.0", x[:n], 5), want[:n]), n
+
+
+@pytest.fixture(scope="module")
+def wide_head_voc():
+    """Heads of 64, the shipped layout's."""
+    c = dataclasses.replace(V.tiny(), n_heads=2)
+    w = V.VocWeights(c, seed=13)
+    say("[gpu] vocoder, heads of 64")
+    g = V.VocDevice(c, w)
+    yield c, w, g, orc.VocOracle(c, w, threads=8)
+    g.close()
+
+
+@pytest.mark.parametrize("n", [63, 71, 241])
+def test_pre_transformer_attention_heads_of_64(wide_head_voc, n):
+    """One query row per wave (63), two with a last workgroup of spare rows
+    (71, 241) and several 64-key tiles, against the oracle."""
+    c, w, g, o = wide_head_voc
+    width = o.stages(codes_for(2, 1), 0)["input_proj"].shape[1]
+    x = (np.random.default_rng(n).standard_normal((n, width)) * 0.5).astype(np.float32)
+    say(f"[gpu] pre_tfm.0, heads of 64, {n} rows")
+    mx, rms = rel_err(g.run_stage("pre_tfm.0", x, 19), o.run_stage("pre_tfm.0", x, 19))
+    assert mx <= STAGE_TOL_MAX and rms <= STAGE_TOL_RMS, (mx, rms)
+
+
+def test_pre_transformer_attention_forms_agree_heads_of_64(wide_head_voc):
+    """As above: 9,000 rows run one wave per row; 65 to 3,904 rows two query
+    rows per wave, 4,100 and 7,000 one, as up to 64 again."""
+    c, w, g, o = wide_head_voc
+    width = o.stages(codes_for(2, 1), 0)["input_proj"].shape[1]
+    x = (np.random.default_rng(78).standard_normal((9000, width)) * 0.5).astype(np.float32)
+    say("[gpu] pre_tfm.0, heads of 64, 9000 rows")
+    want = g.run_stage("pre_tfm.0", x, 5)
+    for n in (1, 64, 65, 71, 127, 129, 241, 3900, 4100, 7000):
+        say(f"[gpu] pre_tfm.0, heads of 64, {n} rows")
         assert np.array_equal(g.run_stage("pre_tfm.0", x[:n], 5), want[:n]), n
 
 
