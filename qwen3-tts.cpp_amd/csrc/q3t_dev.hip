@@ -1656,20 +1656,25 @@ void row_scales(q3t_dev * c, const float * x, int xs, int K, int n, float * out)
 }
 
 // ---------------------------------------------------------- short prefills
-// Up to kRowsMax prompt rows of a Q8_0 model take the multi-stream decode's
-// layer program, the rows of the one prompt in the place of the streams: four
-// few-row GEMMs (RMSNorm, quantisation, residual and SwiGLU inside), the K/V
-// rows, and the 16-wave decode attention with one workgroup per (row, head),
-// 6 launches a layer instead of 11, the same numbers.  Bound by its chain of
-// launches; each 16-row tile adds its weights' fp64 scale work.  Measured on
-// the 0.6B shapes (ms, this / the tiled prefill / GEMV chunks), no history:
-// 2 rows 1.39 / 4.27 / 1.17, 3 rows 1.39 / 4.29 / 2.06, 10 rows 1.44 / 4.34 /
-// 5.80, 32 rows 2.08 / 4.56 / 18.5, 64 rows 3.42 / 4.93 / 37.3; behind 1,000
-// cached positions: 2 rows 1.77 / 8.02 / 2.88, 10 rows 1.81 / 8.02 / 10.7,
-// 64 rows 4.84 / 7.70 / 63.2.  The GEMM's column tiles end at 64 rows; two
-// 64-row passes would take 6.8 ms where the tiled prefill of 96 rows takes 5.3.
-constexpr int kRowsMax = 64;
+// Few prompt rows of a Q8_0 model take the multi-stream decode's layer program,
+// the rows of the one prompt in the place of the streams: four few-row GEMMs
+// (RMSNorm, quantisation, residual and SwiGLU inside), the K/V rows, and the
+// 16-wave decode attention with one workgroup per (row, head), 6 launches a
+// layer instead of 11, the same numbers.  Bound by its chain of launches; each
+// 16-row tile adds its weights' fp64 scale work, where the tiled prefill costs
+// about the same up to 63 rows, but its row attention 3.8 us a cached position
+// (this 0.4 to 1.4).  So up to 16 rows take it, and more, per 16-row tile, from
+// the history on that makes up for the tile.  Measured on the 0.6B shapes (ms,
+// this / the tiled prefill / GEMV chunks), no history: 2 rows 1.39 / 1.63 /
+// 1.17, 3 rows 1.40 / 1.67 / 2.07, 16 rows 1.50 / 1.77 / 9.28, 17 rows 1.98 /
+// 1.79, 40 rows 2.72 / 1.86, 64 rows 3.40 / 2.28; 24 rows behind 30 positions
+// 2.03 / 1.94, behind 100 2.05 / 2.20; 40 rows behind 250 3.00 / 2.78, behind
+// 400 3.09 / 3.34; 56 rows behind 500 4.05 / 3.79, behind 700 4.18 / 4.54; 10
+// rows behind 1,000 1.82 / 5.46 / 10.9.  From 64 rows on the tiled prefill's
+// attention is on MFMA too: 64 rows behind 1,000 4.84 / 3.52.
+constexpr int kRowsMax = 64;    // rows of the few-row GEMMs (four 16-row tiles)
 constexpr int kRowsTwo = 160;   // 2 rows: from this many cached positions (GEMV chunks add 1.7 us each, this 0.4)
+constexpr int kRowsPast[kRowsMax / 16] = {0, 60, 320, 600};   // least history for 1 .. 16, 17 .. 32, ... rows
 
 // Call sites of the short prefill and of the text projection: each has its
 // own tickets and partials (a site's launches all split K alike).
@@ -1733,11 +1738,12 @@ int rows_check(q3t_dev * c) {
     return fail(c, "short prefill: a split-K partial never arrived (device wait timed out)");
 }
 
-// Which prefills take it: all layers Q8_0, at most kRowsMax rows, and an
-// attention launch whose LDS holds a row's scores.  Q3T_PREFILL_MFMA (either
-// value) keeps the other paths.
+// Which prefills take it: all layers Q8_0, less than 64 rows behind enough
+// history, and an attention launch whose LDS holds a row's scores.
+// Q3T_PREFILL_MFMA (either value) keeps the other paths.
 bool rows_prefill(q3t_dev * c, int n, int n_past) {
-    if (n < (n_past < kRowsTwo ? 3 : 2) || n > kRowsMax || std::getenv("Q3T_PREFILL_MFMA") || !c->gqa_lds_ok)
+    if (n < (n_past < kRowsTwo ? 3 : 2) || n >= pf::kAT || n_past < kRowsPast[(n - 1) / 16] ||
+        std::getenv("Q3T_PREFILL_MFMA") || !c->gqa_lds_ok)
         return false;
     const q3t_config & g = c->cfg;
     if (g.head_dim != kHD || g.n_head % g.n_kv_head || g.hidden_size % (4 * ms::kRows)) return false;
@@ -1752,13 +1758,15 @@ bool rows_prefill(q3t_dev * c, int n, int n_past) {
 }
 
 // Which tiled path the talker prefill of n tokens takes: 1 = int8 MFMA GEMMs
-// (Q8_0 layers), 2 = exact F16 VALU GEMMs (F16 layers), 0 = the chunked GEMV
+// (Q8_0 layers), 2 = the F16 GEMMs (F16 layers), 0 = the chunked GEMV
 // prefill.  Short Q8_0 prefills go elsewhere first (rows_prefill).  Tiled needs
 // GEMM-friendly widths and, measured on the 0.6B shapes, pays from 9 rows for
-// Q8_0 (10 rows: 4.3 ms against 5.8 ms in 4-row GEMV chunks) and from 40 rows
-// for F16 (its VALU tiles take ~22 ms for any n up to
-// 64, the GEMV ~2.3 ms per 4 rows).  Q3T_PREFILL_MFMA=0 disables it, =1 uses
-// it for any n.
+// Q8_0 with any history (10 rows 1.7 ms against 5.8 ms in 4-row GEMV chunks; 3
+// rows 1.7 against 2.1, but behind 1,000 positions 5.4 against 4.2).  F16 rows
+// up to 39 stay with the GEMV (22.6 ms at 39 rows), whose sums are exact; from
+// 40 on they take the fast forms (2.1 ms) or, with Q3T_PF_EXACT, the exact
+// tiles (10 ms at 40 and 64 rows).  Q3T_PREFILL_MFMA=0 disables it, =1 uses it
+// for any n.
 int tiled_prefill(q3t_dev * c, int n) {
     const char * e = std::getenv("Q3T_PREFILL_MFMA");
     if (e && e[0] == '0') return 0;
@@ -2181,7 +2189,7 @@ int prefill_mfma(q3t_dev * c, int n, int n_past) {
     return 0;
 }
 
-// Talker prefill of n <= kRowsMax tokens (rows in c->stage) on the few-row
+// Talker prefill of n < kRowsMax tokens (rows in c->stage) on the few-row
 // GEMMs; buffers and outputs as prefill_mfma.
 int prefill_rows(q3t_dev * c, int n, int n_past) {
     const q3t_config & g = c->cfg;
@@ -2279,8 +2287,8 @@ struct ProjWork {
 
 // 2 to kRowsMax ids of Q8_0 text tensors take the few-row GEMMs: two launches,
 // the bias and the SiLU in their epilogues.  Measured (0.6B shapes, us a
-// call, this / tiled / GEMV chunks): 2 ids 45 / 110 / 45, 9 ids 46 / 119 / 138,
-// 32 ids 57 / 124 / 343, 64 ids 80 / 130 / 629; 65 ids tiled 133.
+// call, this / tiled / GEMV chunks): 2 ids 45 / 73 / 45, 9 ids 48 / 81 / 137,
+// 32 ids 59 / 86 / 344, 64 ids 78 / 91 / 635; 65 ids tiled 93.
 bool text_proj_few(const q3t_dev * c, int n) {
     return n >= 2 && n <= kRowsMax && !std::getenv("Q3T_PREFILL_MFMA") && c->fc1.type == Q3T_TYPE_Q8_0 &&
            c->fc2.type == Q3T_TYPE_Q8_0 && rows_site_ok(c->cfg, R_FC1) && rows_site_ok(c->cfg, R_FC2);

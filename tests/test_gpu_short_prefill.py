@@ -1,8 +1,8 @@
 """Short Q8_0 prefills and text projections on the few-row GEMMs.
 
-From 2 to 64 rows a Q8_0 model's prefill and text projection run on the
-multi-stream decode's few-row kernels (16-row activation tiles, K split over
-workgroups).  Sums are exact fp64 sums rounded once, so every row equals the
+A Q8_0 model's prefill of 3 to 16 rows (2 to 63 behind enough history) and its
+text projection of 2 to 64 ids run on the multi-stream decode's few-row
+kernels (16-row activation tiles, K split over workgroups).  Sums are exact fp64 sums rounded once, so every row equals the
 tiled prefill's and the GEMV's bit for bit; the row counts are the edges of
 the 16-row tiles and of the range.
 """
@@ -62,6 +62,32 @@ def test_short_prefill_equals_other_paths(model, monkeypatch, kv, past):
         for other in got[1:]:
             for a, b in zip(got[0], other):
                 assert np.array_equal(a, b), (n, float(np.abs(a - b).max()))
+
+
+@pytest.mark.parametrize("n,past", [(17, 59), (17, 60), (32, 60), (33, 319), (33, 320), (48, 320), (49, 599), (49, 600),
+                                    (63, 600), (64, 600)])
+def test_short_prefill_on_both_sides_of_its_lines(model, monkeypatch, n, past):
+    """More than 16 rows take the few-row GEMMs from 60, 320 or 600 cached positions on, by 16-row tiles."""
+    cfg, dev = model
+    dev.kv_set_type(1)
+    dev.kv_reserve(past + n + 1)
+    rng = np.random.default_rng(past + n)
+    kv = rng.standard_normal((2, past, cfg.n_kv_head, cfg.head_dim)).astype(np.float16)
+    for layer in range(cfg.n_layers):
+        dev.kv_write(layer, kv[0], kv[1])
+    rows = (rng.standard_normal((n, cfg.hidden_size)) * 0.05).astype(np.float32)
+    step = (rng.standard_normal(cfg.hidden_size) * 0.05).astype(np.float32)
+    got = []
+    for env in (None, "1", "0"):
+        if env is None:
+            monkeypatch.delenv("Q3T_PREFILL_MFMA", raising=False)
+        else:
+            monkeypatch.setenv("Q3T_PREFILL_MFMA", env)
+        say(f"[gpu] prefill of {n} rows at {past}, path {env}")
+        got.append(dev.prefill(rows, past) + dev.talker_step(step, past + n))
+    for other in got[1:]:
+        for a, b in zip(got[0], other):
+            assert np.array_equal(a, b), float(np.abs(a - b).max())
 
 
 def test_short_text_projection_equals_other_paths(model, monkeypatch):
