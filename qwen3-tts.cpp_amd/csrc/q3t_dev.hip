@@ -2005,8 +2005,10 @@ bool pf_att_f64() {
 // in the layer's cache) into c->pf_att; fast, into the fp16 rows c->pf_h.  From
 // 64 rows on: fast, one kernel on fp16 (bfloat16) MFMA with fp32 accumulation,
 // else the exact MFMA kernels (scores, softmax, P.V; Q3T_PF_ATT_MFMA=0 keeps
-// the row kernel); below, or when the exact kernels' scores would not fit 4 GiB,
-// one workgroup per row.
+// the row kernel).  Below 64 rows, or where a call's scores and probabilities
+// would pass 4 GiB (16 heads: 6,690 rows), one workgroup per row with fp64 sums:
+// the limit is the exact kernels', but fast calls past it have those sums too
+// and keep them.
 int pf_attention(q3t_dev * c, const LayerDev & L, const uint16_t * kc, const uint16_t * vc, int n, int n_past,
                  bool fast) {
     const q3t_config & g = c->cfg;

@@ -105,6 +105,38 @@ def test_flash_probabilities_are_normalised_then_rounded(monkeypatch, past, n, k
     assert wrong == 0, f"{wrong} of {got.size} values"
 
 
+@pytest.mark.parametrize("which,value", [("k", np.inf), ("k", -np.inf), ("k", np.nan), ("v", np.inf), ("v", np.nan)])
+def test_flash_attention_of_values_that_are_not_finite(monkeypatch, which, value):
+    """One such value in the cached history of one layer: the rows that are not finite are the exact form's (an
+    infinite key turns into a score of either sign, and a row of the one sign has no weight there), the others
+    within the bound of the fp16 rows above."""
+    cfg = qcfg.tiny(n_layers=1)
+    past, n = 70, 130
+    rng = np.random.default_rng(11)
+    kv = rng.standard_normal((2, past, cfg.n_kv_head, cfg.head_dim)).astype(np.float16)
+    kv["kv".index(which), 33, 0, 5] = value
+    rows = (rng.standard_normal((n, cfg.hidden_size)) * 0.05).astype(np.float32)
+    dev = Device(cfg)
+    try:
+        dev.upload_weights(Weights(cfg, "f16", seed=47))
+        dev.kv_reserve(past + n)
+        dev.kv_write(0, kv[0], kv[1])
+        out = {}
+        for exact in ("1", "0"):
+            monkeypatch.setenv("Q3T_PF_EXACT", exact)
+            say(f"[gpu] {which} = {value} in the cache, exact {exact}")
+            out[exact] = dev.prefill(rows, past)[0].astype(np.float64)
+    finally:
+        dev.close()
+    finite = np.isfinite(out["1"]).all(axis=1)
+    assert np.array_equal(np.isfinite(out["0"]).all(axis=1), finite)
+    assert np.isnan(out["0"][~finite]).all() and (~finite).any()
+    if which == "k" and not np.isnan(value):
+        assert finite.any()
+        rel = np.abs(out["0"] - out["1"])[finite].max(axis=1) / np.abs(out["1"][finite]).max(axis=1)
+        assert 0 < rel.max() <= 2.0**-8, rel.max()
+
+
 @pytest.mark.parametrize("n", [65, 1100])
 def test_fast_form_of_one_head(monkeypatch, n):
     """One head: the output projection's K of 128 is half of the four stages that the small tiles hold
