@@ -7,9 +7,11 @@
 // digit pairs a + b = g of int8 dot products: 16 v_mfma_i32_16x16x64_i8 per
 // 64 terms, exact in int32, against 16 v_mfma_f64_16x16x4f64 of 66 clocks
 // (the int8 ones take 18) and two conversions per operand element.  The seven
-// G_g are put together in fp64 and rounded to fp32 once, so the rows equal
-// the f64 forms' (k_att_scores, k_att_pv), whose products and sums are exact
-// too.  Per layer at 1,600 rows of the 0.6B shapes (16 heads): scores 151 -> 51
+// G_g are put together in fp64 and rounded to fp32 once.  The f64 forms
+// (k_att_scores, k_att_pv) add exact products in fp64, so the results are the
+// same bits wherever both sums are exact (their terms and partial sums span 53
+// bits or less), and otherwise unless an fp64 rounding lands on a tie of the
+// fp32 one, about one in 2^28; so too the softmax's sums (below).  Per layer at 1,600 rows of the 0.6B shapes (16 heads): scores 151 -> 51
 // us, P.V 153 -> 52 us; at 209 rows 21 -> 11 and 18 -> 10 us; the softmax that
 // writes digits 27 -> 36 us and the split 15 us where k_att_q took 7.  2,048
 // rows would be 31 us of MFMA time per kernel; the rest is the K / V / P tiles'
@@ -230,7 +232,9 @@ __global__ __launch_bounds__(kAttT, 2) void k_att_scores_int(AttInt a, float sca
 // One row held in registers, RQ groups of four consecutive positions per lane:
 // softmax_row_reg with the probabilities' digits written over the row's own
 // scores, [4 planes][ls] bytes (zeros from cnt to jend, the end of the last
-// tile that k_att_pv_int reads).
+// tile that k_att_pv_int reads).  The same exponentials in another order of the
+// fp64 sum (there a lane has every 64th position): its last bits may differ,
+// and the fp32 reciprocal where they meet a tie.
 template <int RQ>
 __device__ __forceinline__ void softmax_row_digits(float * sr, int cnt, int jend, int ls, int lane) {
     float4 v[RQ];

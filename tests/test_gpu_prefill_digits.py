@@ -1,8 +1,9 @@
 """The tiled prefill's exact attention on int8 digit planes.
 
 Cached fp16 values below 127 are four base-256 digits, and the digit sums are
-put together in fp64 and rounded once, so rows equal the f64 forms'
-(Q3T_PF_ATT_INT=0) bit for bit at every length; a cache with larger values or
+put together in fp64 and rounded once, as the f64 forms' (Q3T_PF_ATT_INT=0)
+are: the same bits at every length, but for an fp64 rounding that meets a tie
+of the fp32 one (about one in 2^28, none in these rows); a cache with larger values or
 infinities runs the f64 bodies of the same kernels.  Row counts are the edges
 of the 64-row tiles, odd tile counts (the dealt-out middle tile) and the row
 lengths where the softmax changes its register count.
