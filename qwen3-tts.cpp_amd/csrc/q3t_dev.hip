@@ -2093,8 +2093,8 @@ int pf_attention(q3t_dev * c, const LayerDev & L, const uint16_t * kc, const uin
 
 // Talker prefill of n tokens (rows in c->stage) with F16 layers: by default on
 // the fast fp16-MFMA GEMMs (fp32 accumulation, the inputs written as fp16
-// rows by the RMSNorm, a rounding pass over the attention rows, and the
-// SwiGLU's two-plane form for the widened ffn_down); with Q3T_PF_EXACT=1
+// rows by the RMSNorm, the attention kernel, and the SwiGLU's two-plane form
+// for the widened ffn_down); with Q3T_PF_EXACT=1
 // on the exact f64-MFMA GEMMs, whose rows equal the GEMV path's.  Same layer
 // program and buffers as prefill_mfma (c->pf_f holds the RMSNorm'd rows of
 // the exact form until SwiGLU overwrites it).
