@@ -88,8 +88,9 @@ struct q3t_dev {
     float * pf_xa = nullptr, * pf_xb = nullptr, * pf_qkv = nullptr, * pf_att = nullptr;
     // f64 MFMA prefill attention: scores and probabilities [n_head][n][ls]
     float * pf_s = nullptr; uint16_t * pf_p = nullptr; size_t pf_sp_cap = 0;
-    // the digit planes of q, K and V of one layer's attention, and the number
-    // of the last attention call whose values did not fit them
+    // the digit planes of q, K and V of one layer's attention (fast F16: its q rows
+    // and V^T tiles), and the number of the last attention call whose values did
+    // not fit the digits
     int8_t * pf_dig = nullptr; size_t pf_dig_cap = 0;
     int32_t * pf_wide = nullptr; int32_t pf_call = 0;
     float * pf_g = nullptr, * pf_u = nullptr, * pf_f = nullptr;

@@ -1,8 +1,8 @@
 """The fast attention of the tiled F16 prefill (scores, softmax and P.V in one kernel) and its GEMM tiles.
 
 Its rows against the exact form's (Q3T_PF_EXACT=1) over the edges of the 64-row and 64-position tiles, behind
-cached positions whose keys grow or shrink with the position, so that the running maximum rises in every tile or
-never again, and with a bfloat16 cache.  Tolerance: the probabilities are rounded to 11 bits (bfloat16: 8), each
+cached positions whose keys grow or shrink with the position, so that a row's weight lies late or early in its
+sweep, and with a bfloat16 cache.  Tolerance: the probabilities are rounded to 11 bits (bfloat16: 8), each
 GEMM input to 11, so a row moves by a few 2^-12 (2^-9) of its largest value per layer; two layers, with room for
 the sums' own spread, stay within 2^-8 (2^-6).  The second layer's q comes from sums that the two forms round
 differently, and a q element that falls the other way moves by 2^-10 (2^-7) of itself: against the grown keys (up
