@@ -1675,7 +1675,11 @@ void row_scales(q3t_dev * c, const float * x, int xs, int K, int n, float * out)
 // attention is on MFMA too: 64 rows behind 1,000 4.84 / 3.52.
 constexpr int kRowsMax = 64;    // rows of the few-row GEMMs (four 16-row tiles)
 constexpr int kRowsTwo = 160;   // 2 rows: from this many cached positions (GEMV chunks add 1.7 us each, this 0.4)
-constexpr int kRowsPast[kRowsMax / 16] = {0, 60, 320, 600};   // least history for 1 .. 16, 17 .. 32, ... rows
+// Least history for 1 .. 16, 17 .. 32, ... rows of the 0.6B layers (15.7 million weights each); a tile's work
+// grows with the layer's weights, and the line with it.  1.7B layers (50.3 million: 192, 1,024, 1,920): 17 rows
+// behind 60 positions 3.30 / 2.83, behind 200 3.35 / 3.35; 48 rows behind 600 5.94 / 5.10; 63 behind 1,000 8.14 / 6.70.
+constexpr int kRowsPast[kRowsMax / 16] = {0, 60, 320, 600};
+constexpr int64_t kRowsWeights = 15728640;
 
 // Call sites of the short prefill and of the text projection: each has its
 // own tickets and partials (a site's launches all split K alike).
@@ -1743,10 +1747,11 @@ int rows_check(q3t_dev * c) {
 // history, and an attention launch whose LDS holds a row's scores.
 // Q3T_PREFILL_MFMA (either value) keeps the other paths.
 bool rows_prefill(q3t_dev * c, int n, int n_past) {
-    if (n < (n_past < kRowsTwo ? 3 : 2) || n >= pf::kAT || n_past < kRowsPast[(n - 1) / 16] ||
-        std::getenv("Q3T_PREFILL_MFMA") || !c->gqa_lds_ok)
+    if (n < (n_past < kRowsTwo ? 3 : 2) || n >= pf::kAT || std::getenv("Q3T_PREFILL_MFMA") || !c->gqa_lds_ok)
         return false;
     const q3t_config & g = c->cfg;
+    const int64_t weights = (int64_t) g.hidden_size * ((2 * g.n_head + 2 * g.n_kv_head) * g.head_dim + 3 * g.ffn_size);
+    if (n_past * kRowsWeights < kRowsPast[(n - 1) / 16] * weights) return false;
     if (g.head_dim != kHD || g.n_head % g.n_kv_head || g.hidden_size % (4 * ms::kRows)) return false;
     for (int s : {(int) R_QKV, (int) R_WO, (int) R_GATE_UP, (int) R_DOWN})
         if (!rows_site_ok(g, s)) return false;

@@ -64,11 +64,14 @@ def test_short_prefill_equals_other_paths(model, monkeypatch, kv, past):
                 assert np.array_equal(a, b), (n, float(np.abs(a - b).max()))
 
 
-@pytest.mark.parametrize("n,past", [(17, 59), (17, 60), (32, 60), (33, 319), (33, 320), (48, 320), (49, 599), (49, 600),
-                                    (63, 600), (64, 600)])
-def test_short_prefill_on_both_sides_of_its_lines(model, monkeypatch, n, past):
-    """More than 16 rows take the few-row GEMMs from 60, 320 or 600 cached positions on, by 16-row tiles."""
+@pytest.mark.parametrize("side", [-1, 0])
+@pytest.mark.parametrize("n,line", [(17, 60), (32, 60), (33, 320), (48, 320), (49, 600), (63, 600), (64, 600)])
+def test_short_prefill_on_both_sides_of_its_lines(model, monkeypatch, n, line, side):
+    """More than 16 rows take the few-row GEMMs from `line` cached positions on, times the layer's weights over the
+    15,728,640 of the 0.6B layers; 64 rows never."""
     cfg, dev = model
+    weights = cfg.hidden_size * ((2 * cfg.n_head + 2 * cfg.n_kv_head) * cfg.head_dim + 3 * cfg.ffn_size)
+    past = -(-line * weights // 15728640) + side
     dev.kv_set_type(1)
     dev.kv_reserve(past + n + 1)
     rng = np.random.default_rng(past + n)
